@@ -36,9 +36,12 @@ BF16_DENSE_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
 INT8_DENSE_TOPS = 5000.0     # MI355X dense int8 MFMA
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_mx_mfma_decode_b64_36layers.md")
 MFMA_PROFILE = os.path.join(ROOT, "profiles", "k_mx_gemm_prefill_b512_hot.md")
-# grouped-GEMM policy of the library's default (spt_abi.hip: kGemmMinGroup,
-# kGemmMinSelections; select: items must fill half the device)
-GEMM_MIN_GROUP, GEMM_MIN_SELECTIONS = 9, 384
+# policy of the library's default for the wide launches (spt_abi.hip:
+# kGemmMinGroup, kGemmMinSelections, kGemmMinGain, kGemvMinExperts;
+# spt_kernels.hip: the costs of a wide pass of one and of two tiles and of a
+# GEMV pass)
+GEMM_MIN_GROUP, GEMM_MIN_SELECTIONS, GEMM_MIN_GAIN, GEMV_MIN_EXPERTS = 5, 384, 200, 4
+WIDE_COST1, WIDE_COST2, GEMV_PASS_COST = 25, 37, 14
 # selections per grouped-GEMV weight pass (spt_kernels.h: kGemvTokens)
 GEMV_TOKENS = 4
 # host threads for the CPU baseline: the host's CPU share per GPU
@@ -377,7 +380,12 @@ def prefill(args, ctx, dl, shp, W, stream, reps=20):
         distinct = int(np.count_nonzero(c))
         n = B * k
         big = c[c >= GEMM_MIN_GROUP]
-        gemm_on = n >= GEMM_MIN_SELECTIONS and int(np.sum((big + 63) // 64)) * ((D + 127) // 128) >= 128
+        rem = big % 64
+        wide = big // 64 * WIDE_COST2 + np.where(rem == 0, 0, np.where(rem > 32, WIDE_COST2, WIDE_COST1))
+        gain = int(np.sum((big + GEMV_TOKENS - 1) // GEMV_TOKENS * GEMV_PASS_COST - wide))
+        gemm_on = n >= GEMM_MIN_SELECTIONS and gain >= GEMM_MIN_GAIN and int(np.sum((big + 63) // 64)) * (D // 32) >= 512
+        gemm_min = 1 if int(np.sum((c > 0) & (c < GEMM_MIN_GROUP))) < GEMV_MIN_EXPERTS else GEMM_MIN_GROUP
+        big = c[c >= gemm_min]
         gemm_sel = int(big.sum()) if gemm_on else 0
         # warm for at least 60 ms of back-to-back layers: a few calls after
         # the host-side set-up above the 512-token layer still runs about
@@ -408,7 +416,7 @@ def prefill(args, ctx, dl, shp, W, stream, reps=20):
         wbytes = distinct * (2 * shp.gate_bytes + shp.down_bytes)
         # the grouped GEMV streams each of its experts once per pass of
         # GEMV_TOKENS selections: its weight bytes once, and as streamed
-        gv = c[(c > 0) & ~((c >= GEMM_MIN_GROUP) & gemm_on)]
+        gv = c[(c > 0) & ~((c >= gemm_min) & gemm_on)]
         gv_passes = int(np.sum((gv + GEMV_TOKENS - 1) // GEMV_TOKENS))
         res = {
             "batch": B, "ms_per_layer": round(ms, 4), "tokens_per_s": round(B / (ms / 1e3), 1),

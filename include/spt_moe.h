@@ -128,10 +128,10 @@ int spt_ctx_synchronize(struct spt_ctx *ctx);
 int spt_ctx_set_cancel_flag(struct spt_ctx *ctx, const volatile int32_t *flag);
 
 /* Expert groups of at least min_group selections run through the grouped
- * GEMM (bf16 MFMA, up to 64 selections per pass over the expert's weights);
- * smaller groups through the grouped GEMV (4 per pass).  0 restores the
- * default policy: groups of 9 or more when the batch holds at least 384
- * selections and those groups' GEMM work fills half the device.  Results are the
+ * GEMM (block-scaled MFMA, up to 64 selections per pass over the expert's
+ * weights); smaller groups through the grouped GEMV (4 per pass).  0 restores
+ * the default policy: groups of 5 or more when the batch holds at least 384
+ * selections and the passes saved outweigh the launches.  Results are the
  * same either way within the fp32 tolerance (the per-block sums are exact on
  * both).  No reference counterpart: the reference picks its CPU loop by tile
  * size (forward/mxfp4_batch.go:55-95). */

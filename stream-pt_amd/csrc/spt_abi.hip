@@ -38,11 +38,6 @@ struct spt_ctx {
     int32_t gemm_min_group = 0;  // 0: the default policy (kGemmMinGroup)
     int32_t decode_max_selections = 0;  // 0: kDecodeMaxSelections; < 0: decode path off
     int n_cu = 0;                // compute units of the device
-    // A second stream of the device and two events: a layer's grouped GEMM
-    // launches run there beside its GEMV launches (fork after the
-    // selection, join before the combine).  Null: everything on `stream`.
-    hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
 
 // Scratch of spt_forward_moe_batch_noalloc: a fixed device array, one copy
@@ -341,6 +336,9 @@ int validate_bias(const spt_tensor *t, int64_t dim, int64_t count) {
 
 const void *bias_ptr(const spt_tensor &t) { return named(t) ? t.data : nullptr; }
 int bias_type(const spt_tensor &t) { return named(t) ? (int)t.type : 0; }
+bool elements_aligned(const spt_tensor &t) {
+    return ((uintptr_t)bias_ptr(t) & (bias_type(t) == SPT_TYPE_F32 ? 3u : 1u)) == 0;
+}
 uint64_t bias_bytes(const spt_tensor &t) { return named(t) ? t.nbytes : 0; }
 
 struct MoEDims {
@@ -348,8 +346,8 @@ struct MoEDims {
 };
 
 // forwardMoEBatch validation (forward/moe_batch.go:81-130).  With `sliced`
-// the batch may hold more selections than one launch sequence takes
-// (spt::kMaxSelections): the caller runs it as slices of whole tokens.
+// the batch may hold more selections than spt::kMaxSelections: the caller
+// runs it as slices of whole tokens.
 int validate_moe(spt_ctx *ctx, const spt_moe_config *cfg, const spt_moe_layer *lw,
                  const float *x, int64_t x_len, const float *out, int64_t out_len, int64_t batch,
                  MoEDims *dims, bool sliced = false) {
@@ -397,19 +395,24 @@ int copy_tap(spt_ctx *ctx, void *dst, const void *src, size_t bytes) {
     return SPT_OK;
 }
 
-// Default policy for the grouped GEMM (measured on MI355X with GPT-OSS
-// shapes): groups of at least kGemmMinGroup selections (three or more GEMV
-// passes over the expert's weights) go to the GEMM when the batch holds at
-// least kGemmMinSelections selections and their work items fill at least
-// half the device; below that the GEMV's passes are faster (a GEMM item
-// walks the whole input dimension serially, and the persistent GEMV holds
-// every CU until it ends, so a few GEMM items run after it as a tail).
-// Measured per layer, Zipf(1.1) routing, default against GEMV only: 96
-// tokens 299 / 322 us, 128: 338 / 373, 160: 379 / 483, 192: 392 / 545;
-// uniform routing at 96 and 128 tokens (one or two groups of 9 or 10) stays
-// on the GEMV (328, 400 us; 386, 457 with those groups on the GEMM).
-constexpr int kGemmMinGroup = 9;
+// Default policy for the wide product (spt_mx_wide.hip; measured on MI355X
+// with GPT-OSS shapes, us per layer): a group of one GEMV pass (up to four
+// selections) stays on the GEMV, which streams weights faster; larger groups
+// go to the wide launches, which read an expert's weights once per 64
+// selections, when the batch holds at least kGemmMinSelections selections and
+// the passes saved are worth more than the two launches (kGemmMinGain, about
+// 20 us of gate/up) and make two units or more for each workgroup.  GEMV only / thresholds of 9 / 5: uniform routing 96
+// tokens 354 / 363 / 359, 128: 436 / 432 / 414, 256: 721 / 567 / 536; Zipf(1.1)
+// 96: 284 / 207 / 204, 256: 654 / 309 / 307.  Below 384 selections the wide
+// launches' fixed cost outweighs the passes they save (Zipf(0.6): 48 tokens
+// 204 / 231 / 229, 64: 240 / 256 / 254).  With fewer than kGemvMinExperts
+// small groups these go to the wide launches too: a GEMV launch for a few
+// experts costs more than their share of the wide ones (uniform, 512 tokens:
+// 592 with five experts on the GEMV, 569 without).
+constexpr int kGemmMinGroup = 5;
 constexpr int kGemmMinSelections = 384;
+constexpr int kGemmMinGain = 200;
+constexpr int kGemvMinExperts = 4;
 // Batches of up to this many selections (topk <= 4, no GEMM group) take the
 // decode path: top-k inside the gate/up launch, combine inside the down
 // launch, a workgroup per selection (spt_mx_decode.hip).  Measured on the
@@ -426,37 +429,38 @@ struct MoELayout {
     int gemm_min;
     bool forced;
     size_t o_xc, o_xs, o_xm, o_xb, o_logits, o_ids, o_w, o_cnt, o_off, o_list, o_act_list, o_na;
-    size_t o_gv, o_gvn, o_gvp, o_gvs, o_gm, o_gmn, o_gmt, o_act, o_ac, o_as, o_am, o_ab, o_res;
+    size_t o_gv, o_gvn, o_gvp, o_gvs, o_gm, o_gms, o_act, o_ac, o_as, o_am, o_ab, o_res;
     size_t total;
 };
 
 // An expert's group holds at most n selections: with fewer than the
-// threshold no expert can reach the GEMM, which is then not launched.  An
-// explicit threshold (spt_ctx_set_gemm_min_group) applies as given; the
-// default also needs kGemmMinSelections and half a device of items.  The
-// fp32 act buffer exists only for the act tap.
+// threshold no expert can reach the wide launches, which are then left out.
+// An explicit threshold (spt_ctx_set_gemm_min_group) applies as given; the
+// default also needs kGemmMinSelections.  The fp32 act buffer exists only
+// for the act tap.
 MoELayout moe_layout(const spt_ctx *ctx, const MoEDims &m, bool act_tap, size_t base) {
     const int64_t h = m.h, d = m.d, E = m.E, B = m.batch, n = m.batch * m.k;
     const int64_t nbh = h / 32, nbd = d / 32;
     MoELayout L{};
     L.forced = ctx->gemm_min_group > 0;
     L.gemm_min = L.forced ? ctx->gemm_min_group : kGemmMinGroup;
-    L.use_gemm = n >= L.gemm_min && (L.forced || n >= kGemmMinSelections);
+    L.use_gemm = n >= L.gemm_min && (L.forced || n >= kGemmMinSelections) && spt::mx_wide_grid() <= spt::kGvStartMax;
     const int dec_max = ctx->decode_max_selections == 0 ? kDecodeMaxSelections : ctx->decode_max_selections;
     L.decode = !L.use_gemm && m.k <= spt::kDecMaxTopK && n <= dec_max;
     Carve c;
     c.off = base;
     L.o_xc = c.take(B * h), L.o_xs = c.take(B * nbh * 4), L.o_xm = c.take(B * nbh * 64);
-    L.o_xb = c.take(L.use_gemm ? B * nbh * 64 : 0);
+    L.o_xb = c.take(L.use_gemm ? B * nbh * spt::kDigitBytes : 0);
     L.o_logits = c.take(B * E * 4);
     L.o_ids = c.take(n * 4), L.o_w = c.take(n * 4), L.o_cnt = c.take(E * 4), L.o_off = c.take((E + 1) * 4);
     L.o_list = c.take(n * 4), L.o_act_list = c.take(E * 4), L.o_na = c.take(4);
     L.o_gv = c.take(E * 4), L.o_gvn = c.take(4), L.o_gvp = c.take((E + 1) * 4);
     L.o_gvs = c.take(L.decode ? 0 : sizeof(int32_t) * 2 * spt::kGvStartMax * spt::kGvStartWords);
-    L.o_gm = c.take(E * 4), L.o_gmn = c.take(12), L.o_gmt = c.take((E + 1) * 4);  // gm_n, then the two claim counters
+    L.o_gms = c.take(L.decode ? 0 : sizeof(int32_t) * 2 * spt::kGvStartMax * spt::kGvStartWords);
+    L.o_gm = c.take(E * 4);
     L.o_act = c.take(act_tap ? n * d * 4 : 0), L.o_ac = c.take(n * d), L.o_as = c.take(n * nbd * 4);
     L.o_am = c.take(n * nbd * 64);
-    L.o_ab = c.take(L.use_gemm ? n * nbd * 64 : 0);
+    L.o_ab = c.take(L.use_gemm ? n * nbd * spt::kDigitBytes : 0);
     L.o_res = c.take(L.decode ? 0 : n * h * 4);  // the decode path combines in its down launch
     L.total = c.off;
     return L;
@@ -468,14 +472,19 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
                const spt_moe_taps *taps, char *S, const MoELayout &L, const uint8_t *xq34 = nullptr) {
     const int64_t h = m.h, d = m.d, E = m.E, k = m.k, B = m.batch, n = B * k;
     const int64_t nbh = h / 32, nbd = d / 32;
-    const bool use_gemm = L.use_gemm, forced = L.forced;
+    // (the wide launches read the biases by whole aligned elements; others
+    // stay with the GEMV)
+    const bool use_gemm = L.use_gemm && spt::mx_wide_fits((uint64_t)nbh * 17 * d) && spt::mx_wide_fits((uint64_t)nbd * 17 * h) &&
+                          elements_aligned(lw->ffn_gate_exps_bias) &&
+                          elements_aligned(lw->ffn_up_exps_bias) && elements_aligned(lw->ffn_down_exps_bias);
+    const bool forced = L.forced;
     const int gemm_min = L.gemm_min;
     int rc;
     int8_t *xc = (int8_t *)(S + L.o_xc), *ac = (int8_t *)(S + L.o_ac);
     float *xs = (float *)(S + L.o_xs), *logits = (float *)(S + L.o_logits);
     float *act = taps && taps->act ? (float *)(S + L.o_act) : nullptr;
     uint8_t *xm = (uint8_t *)(S + L.o_xm), *am = (uint8_t *)(S + L.o_am);
-    uint32_t *xb = use_gemm ? (uint32_t *)(S + L.o_xb) : nullptr, *ab = use_gemm ? (uint32_t *)(S + L.o_ab) : nullptr;
+    uint8_t *xb = use_gemm ? (uint8_t *)(S + L.o_xb) : nullptr, *ab = use_gemm ? (uint8_t *)(S + L.o_ab) : nullptr;
     float *as = (float *)(S + L.o_as), *res = (float *)(S + L.o_res);
     spt::SelectOut so{};
     so.ids = (int32_t *)(S + L.o_ids);
@@ -486,15 +495,19 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     so.active = (int32_t *)(S + L.o_act_list);
     so.n_active = (int32_t *)(S + L.o_na);
     so.gemm_min = use_gemm ? gemm_min : INT_MAX;
-    so.gemm_units = (int32_t)((d + 127) / 128);
-    so.gemm_min_items = forced ? 0 : ctx->n_cu / 2;
+    so.gemm_min_gain = forced ? INT_MIN : kGemmMinGain;
+    so.gemm_min_units = forced ? 0 : 2 * ctx->n_cu;
+    so.gv_min_experts = forced ? 0 : kGemvMinExperts;
     so.gv_active = (int32_t *)(S + L.o_gv);
     so.gv_n = (int32_t *)(S + L.o_gvn);
     so.gv_pass_off = (int32_t *)(S + L.o_gvp);
     so.gm_active = (int32_t *)(S + L.o_gm);
-    so.gm_n = (int32_t *)(S + L.o_gmn);
-    so.gm_claim = (int32_t *)(S + L.o_gmn) + 1;
-    so.gm_tile_off = (int32_t *)(S + L.o_gmt);
+    if (use_gemm) {
+        so.gm_start = (int32_t *)(S + L.o_gms);
+        so.gm_grid = spt::mx_wide_grid();
+        so.wide_units[0] = (int32_t)(d / spt::kWideRows);
+        so.wide_units[1] = (int32_t)(h / spt::kWideRows);
+    }
     // the two grouped GEMV launches' start table, for their grids
     const int slots = (int)(n < E ? n : E);
     if (!L.decode) {
@@ -516,7 +529,7 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     if ((rc = check_cancel(ctx))) return rc;
     if (taps && taps->logits_in) {
         SPT_HIP(timed(ctx, SPT_KERNEL_QUANTIZE, [&] {
-            return spt::launch_quantize(s, x, B * nbh, xq.codes, xq.scales, nullptr, xq.mxtab, xq.blocks34, xq.btab);
+            return spt::launch_quantize(s, x, B * nbh, xq.codes, xq.scales, nullptr, xq.mxtab, xq.blocks34, xq.dtab);
         }));
         if (!L.decode)
             SPT_HIP(timed(ctx, SPT_KERNEL_SELECT, [&] { return spt::launch_select(s, taps->logits_in, (int)B, (int)E, (int)k, so); }));
@@ -630,50 +643,30 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     ga.act_blocks34 = taps ? (uint8_t *)taps->actq : nullptr;
     ga.start = so.gv_start;
     if ((rc = check_cancel(ctx))) return rc;
-    // The grouped GEMM (its own experts, act rows and results) on the side
-    // stream from here to the combine, so its launches fill the CUs the
-    // GEMV launches leave idle and the reverse; with timing on, in line.
-    // The join is recorded however the call ends.
-    struct Join {
-        spt_ctx *ctx;
-        hipStream_t s;
-        bool on = false;
-        ~Join() {
-            if (on && hipEventRecord(ctx->ev_join, ctx->side) == hipSuccess)
-                (void)hipStreamWaitEvent(s, ctx->ev_join, 0);
-        }
-    } join{ctx, s};
-    hipStream_t sg = s;
-    if (use_gemm && ctx->side && !ctx->timing) {
-        SPT_HIP(hipEventRecord(ctx->ev_fork, s));
-        SPT_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-        sg = ctx->side;
-        join.on = true;
-    }
+    // The GEMV's experts, then the wide launches' (their own act rows and
+    // results), one after the other: both deal their work to one workgroup
+    // per compute unit in equal shares, and beside each other on two streams
+    // the workgroups that come second on a unit finish late (uniform routing,
+    // 206 tokens, 32 experts: 174 us on two streams, 156 on one; Zipf(1.1)
+    // layers 1-3 % the other way).
     SPT_HIP(timed(ctx, SPT_KERNEL_GATE_UP, [&] { return spt::launch_mx_mfma(s, spt::kGateUp, ga, slots); }));
-    // Upper bound of the GEMM work items (token tiles x row units): every
-    // GEMM expert holds at least gemm_min selections.
-    const int64_t gm_experts = use_gemm ? std::min<int64_t>(E, n / gemm_min) : 0;
-    const int64_t gm_tiles = gm_experts + (n + spt::kGemmTokens - 1) / spt::kGemmTokens;
-    spt::MxGemmArgs gg{};
+    spt::MxWideArgs gg{};
     if (use_gemm) {
         gg.w[0] = ga.w[0];
         gg.w[1] = ga.w[1];
         gg.expert_bytes = ga.expert_bytes;
         gg.rows = ga.rows;
         gg.nb = ga.nb;
-        gg.bias[0] = ga.bias[0];
-        gg.bias[1] = ga.bias[1];
-        gg.bias_type[0] = ga.bias_type[0];
-        gg.bias_type[1] = ga.bias_type[1];
-        gg.btab = xb;
-        gg.tab_rows = B;
-        gg.scales = xs;
+        for (int i = 0; i < 2; i++) {
+            gg.bias[i] = ga.bias[i];
+            gg.bias_bytes[i] = ga.bias_bytes[i];
+            gg.bias_type[i] = ga.bias_type[i];
+        }
+        gg.active = so.gm_active;
+        gg.start = so.gm_start;
+        gg.tab = xb;
+        gg.tab_bytes = (uint32_t)(B * nbh * spt::kDigitBytes);
         gg.codes = xc;
-        gg.gm_active = so.gm_active;
-        gg.gm_n = so.gm_n;
-        gg.claim = so.gm_claim;
-        gg.gm_tile_off = so.gm_tile_off;
         gg.offsets = so.offsets;
         gg.list = so.list;
         gg.topk = (int)k;
@@ -681,15 +674,10 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
         gg.tap[0] = ga.tap[0];
         gg.tap[1] = ga.tap[1];
         gg.act_codes = ac;
-        gg.act_scales = as;
-        gg.act_mxtab = nullptr;  // read only by the GEMV's down pass
+        gg.act_tab = ab;
         gg.act_blocks34 = ga.act_blocks34;
-        gg.act_btab = ab;
-        const int64_t items = gm_tiles * ((d + 127) / 128);
         if ((rc = check_cancel(ctx))) return rc;
-        SPT_HIP(timed(ctx, SPT_KERNEL_GATE_UP_GEMM, [&] {
-            return spt::launch_mx_gemm(sg, spt::kGateUp, gg, (int)std::min<int64_t>(items, INT_MAX));
-        }));
+        SPT_HIP(timed(ctx, SPT_KERNEL_GATE_UP_GEMM, [&] { return spt::launch_mx_wide(s, spt::kGateUp, gg); }));
     }
     spt::MxMfmaArgs da{};
     da.w[0] = (const uint8_t *)lw->ffn_down_exps.data;
@@ -713,35 +701,25 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     if ((rc = check_cancel(ctx))) return rc;
     SPT_HIP(timed(ctx, SPT_KERNEL_DOWN, [&] { return spt::launch_mx_mfma(s, spt::kDown, da, slots); }));
     if (use_gemm) {
-        spt::MxGemmArgs gd{};
+        spt::MxWideArgs gd{};
         gd.w[0] = da.w[0];
         gd.expert_bytes = da.expert_bytes;
         gd.rows = da.rows;
         gd.nb = da.nb;
         gd.bias[0] = da.bias[0];
+        gd.bias_bytes[0] = da.bias_bytes[0];
         gd.bias_type[0] = da.bias_type[0];
-        gd.btab = ab;
-        gd.tab_rows = n;
-        gd.scales = as;
+        gd.active = so.gm_active;
+        gd.start = so.gm_start + spt::kGvStartMax * spt::kGvStartWords;
+        gd.tab = ab;
+        gd.tab_bytes = (uint32_t)(n * nbd * spt::kDigitBytes);
         gd.codes = ac;
-        gd.gm_active = so.gm_active;
-        gd.gm_n = so.gm_n;
-        gd.claim = so.gm_claim + 1;
-        gd.gm_tile_off = so.gm_tile_off;
         gd.offsets = so.offsets;
         gd.list = so.list;
         gd.topk = (int)k;
         gd.out = res;
-        const int64_t items = gm_tiles * ((h + 255) / 256);
         if ((rc = check_cancel(ctx))) return rc;
-        SPT_HIP(timed(ctx, SPT_KERNEL_DOWN_GEMM, [&] {
-            return spt::launch_mx_gemm(sg, spt::kDown, gd, (int)std::min<int64_t>(items, INT_MAX));
-        }));
-    }
-    if (join.on) {
-        join.on = false;
-        SPT_HIP(hipEventRecord(ctx->ev_join, sg));
-        SPT_HIP(hipStreamWaitEvent(s, ctx->ev_join, 0));
+        SPT_HIP(timed(ctx, SPT_KERNEL_DOWN_GEMM, [&] { return spt::launch_mx_wide(s, spt::kDown, gd); }));
     }
     if ((rc = check_cancel(ctx))) return rc;
     SPT_HIP(timed(ctx, SPT_KERNEL_COMBINE, [&] { return spt::launch_combine(s, res, so.weights, (int)B, (int)k, (int)h, out); }));
@@ -760,12 +738,15 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
 }
 
 // Tokens per launch sequence: a batch of more selections than
-// spt::kMaxSelections runs as consecutive slices of this many whole tokens.
-// The reference accepts any batch (forward/moe_batch.go:29-38,84-90), and a
-// token's output depends only on its own row of x, so slicing changes no
-// routing; the slices' own expert groups decide which of the grouped GEMV
-// and GEMM each group takes, as for separate calls of those tokens.
-int64_t moe_slice_tokens(const MoEDims &m) { return spt::kMaxSelections / m.k; }
+// spt::kSliceSelections runs as consecutive slices of this many whole tokens
+// (its arena then holds about 250 MB at GPT-OSS-120B shape).  The reference
+// accepts any batch (forward/moe_batch.go:29-38,84-90), and a token's output
+// depends only on its own row of x, so slicing changes no routing; but every
+// slice streams the weights of all its experts, so slices are as large as the
+// packing kernel's LDS comfortably takes.  The slices' own expert groups
+// decide which of the grouped GEMV and the wide product each group takes, as
+// for separate calls of those tokens.
+int64_t moe_slice_tokens(const MoEDims &m) { return spt::kSliceSelections / m.k; }
 
 int run_moe(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out, const MoEDims &m,
             const spt_moe_taps *taps) {
@@ -1196,17 +1177,6 @@ int spt_ctx_create(int device, void *hip_stream, spt_ctx **out) {
             ctx->n_cu = 256;
         // with the device current: its copy of the no-allocation scratch
         noalloc_scratch_of(device, &ctx->noalloc, &ctx->noalloc_err);
-        // the side stream (default priority) and its fork / join events; if
-        // any of them cannot be made, layers run on the one stream
-        if (hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess) {
-            if (ctx->side) (void)hipStreamDestroy(ctx->side);
-            if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
-            if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
-            ctx->side = nullptr;
-            ctx->ev_fork = ctx->ev_join = nullptr;
-        }
     }
     *out = ctx;
     return SPT_OK;
@@ -1224,12 +1194,6 @@ int spt_ctx_destroy(spt_ctx *ctx) {
             (void)hipEventDestroy(p.second.second);
         }
         for (hipEvent_t e : ctx->free_events) (void)hipEventDestroy(e);
-        if (ctx->side) {
-            (void)hipStreamSynchronize(ctx->side);
-            (void)hipStreamDestroy(ctx->side);
-            (void)hipEventDestroy(ctx->ev_fork);
-            (void)hipEventDestroy(ctx->ev_join);
-        }
         if (ctx->own_stream) (void)hipStreamDestroy(ctx->stream);
     }
     delete ctx;

@@ -55,6 +55,9 @@ __device__ inline void dma16_nt(const u32x4v &rs, uint32_t lds, uint32_t voff, u
 __device__ inline void dma16_other_stage(const u32x4v &rs, uint32_t lds, uint32_t voff, uint32_t soff) {
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds));
 }
+__device__ inline void dma16_nt_other_stage(const u32x4v &rs, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds));
+}
 __device__ inline void dma4(const u32x4v &rs, uint32_t lds, uint32_t voff, uint32_t soff) {
     asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds)
                  : "memory");
@@ -297,71 +300,33 @@ __device__ inline uint32_t e4m3_small(int v) {
     return v < 0 ? (code | 0x80u) : code;
 }
 
-// Store one quantized block of 32 (codes w[8], fp16 scale bits dh) as block
-// `blk` of every requested layout:
-//   codes  : int8 [blk][32]
-//   scales : f32  [blk]          (fp16 d widened exactly)
-//   mxtab  : u8   [blk][64]      E4M3 digits of q = 16*h + l in MXFP4 nibble
-//                                 order (position p <-> element (p>>1) +
-//                                 16*(p&1)): h digits at [0,32), l at [32,64)
-//   blocks34: u8  [blk][34]      GGML Q8_0 block
-//   btab   : u32 [blk][16]       bf16 codes for the bf16 MFMA, dword j =
-//                                 bf16(q[j]) | bf16(q[j+16]) << 16 (the
-//                                 MXFP4 nibble order of bytes 1+j)
-__device__ inline uint32_t bf16_code_pair(int lo, int hi) {
-    return (__float_as_uint((float)lo) >> 16) | (__float_as_uint((float)hi) & 0xFFFF0000u);
+// FP6 E2M3 encoding of a small integer n as the value n / 8 (sign and
+// magnitude), exact for |n| <= 16.
+__device__ inline uint32_t e2m3_small(int v) { return v < 0 ? 32u | (uint32_t)(-v) : (uint32_t)v; }
+
+// The same of the h digits (q >> 4) of four codes q, one per byte: the two's
+// complement nibble looked up by its low three bits in a table for each sign.
+__device__ inline uint32_t e2m3_high4(uint32_t q) {
+    const uint32_t n = (q >> 4) & 0x0F0F0F0Fu, i = n & 0x07070707u;
+    const uint32_t neg = __builtin_amdgcn_perm(0x21222324u, 0x25262728u, i);  // -8 .. -1
+    return __builtin_amdgcn_perm(neg, i, ((n >> 1) & 0x04040404u) | 0x03020100u);
 }
 
-__device__ inline void write_q8_block(const uint32_t w[8], uint16_t dh, size_t blk, int8_t *codes,
-                                      float *scales, uint8_t *mxtab, uint8_t *blocks34,
-                                      uint32_t *btab = nullptr) {
-    if (codes) {
-        uint32_t *c = reinterpret_cast<uint32_t *>(codes + blk * 32);
-#pragma unroll
-        for (int k = 0; k < 8; k++) c[k] = w[k];
-    }
-    if (scales) scales[blk] = f16_bits_to_f32(dh);
-    if (mxtab) {
-        uint32_t hw[8], lw[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            hw[k] = 0;
-            lw[k] = 0;
-        }
-#pragma unroll
-        for (int p = 0; p < 32; p++) {
-            const int el = (p >> 1) + 16 * (p & 1);
-            const int q = (int)(int8_t)(w[el >> 2] >> (8 * (el & 3)));
-            const int h = q >> 4, l = q & 15;
-            hw[p >> 2] |= e4m3_small(h) << (8 * (p & 3));
-            lw[p >> 2] |= e4m3_small(l) << (8 * (p & 3));
-        }
-        uint32_t *o = reinterpret_cast<uint32_t *>(mxtab + blk * 64);
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            o[k] = hw[k];
-            o[8 + k] = lw[k];
-        }
-    }
-    if (blocks34) {
-        uint8_t *o = blocks34 + blk * kQ80Block;
-        o[0] = (uint8_t)(dh & 0xff);
-        o[1] = (uint8_t)(dh >> 8);
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[2 + 4 * k + i] = (uint8_t)(w[k] >> (8 * i));
-    }
-    if (btab) {
-        uint32_t *o = btab + blk * 16;
-#pragma unroll
-        for (int j = 0; j < 16; j++) {
-            const int lo = (int)(int8_t)(w[j >> 2] >> (8 * (j & 3)));
-            const int hi = (int)(int8_t)(w[4 + (j >> 2)] >> (8 * (j & 3)));
-            o[j] = bf16_code_pair(lo, hi);
-        }
-    }
+// Four 6-bit bytes to 24 bits.
+__device__ inline uint32_t pack6x4(uint32_t b) {
+    const uint32_t t = (b & 0x003F003Fu) | ((b >> 2) & 0x0FC00FC0u);
+    return (t & 0xFFFu) | ((t >> 4) & 0xFFF000u);
 }
+
+// Digit table of a Q8_0 block for the 32x32x64 block-scaled MFMA: 64 bytes
+// holding the E2M3 digits of q = 16*h + l in MXFP4 nibble order (position p <->
+// element (p>>1) + 16*(p&1)), 6 bits each, 24 bytes a digit: byte o of digit
+// row g (0: h, 1: l) at digit_byte(g, o), and after the row's last 8 bytes the
+// scale (f32, in both rows), so a lane takes its row and the scale by two
+// 16-byte loads.
+constexpr int kDigitBytes = 64;
+__device__ inline int digit_byte(int g, int o) { return o < 16 ? 16 * g + o : 32 + 16 * g + (o - 16); }
+__device__ inline int digit_scale(int g) { return 40 + 16 * g; }
 
 // The same rule with one element per lane (lanes 0..31 of a wavefront hold
 // the block; lanes 32..63 pass v = 0 and their results are unused).  amax
@@ -411,15 +376,44 @@ __device__ __attribute__((always_inline)) inline int q8_quantize_half(float v, i
     return (r != r) ? 0 : (r > 127.0f ? 127 : (r < -127.0f ? -127 : (int)r));
 }
 
-// Lane i (< 32) of a wavefront stores element i of Q8_0 block `blk` (code q)
-// into every requested layout of write_q8_block; lane 0 also stores the scale.
+// The Q8_0 code of v = x / d: half away from zero, NaN 0, clamped to +-127.
+// Adding the largest float below 0.5 (v's sign) and truncating rounds half
+// away from zero: a v just below a half stays below the next integer.
+__device__ __attribute__((always_inline)) inline int q8_code(float v) {
+    const int q = (int)(v + __builtin_copysignf(0.49999997f, v));  // v_cvt_i32_f32: NaN 0, saturating
+    return max(-127, min(127, q));
+}
+
+// Lane i (< 32) of a half-wave stores element i of Q8_0 block `blk` (code q)
+// into every requested layout; lane 0 also stores the scale.
+//   codes    : int8 [blk][32]
+//   scales   : f32  [blk]      (fp16 d widened exactly)
+//   mxtab    : u8   [blk][64]  E4M3 digits of q = 16*h + l in MXFP4 nibble
+//                              order: h digits at [0,32), l at [32,64)
+//   blocks34 : u8   [blk][34]  GGML Q8_0 block
+//   dtab     : u8   [blk][64]  E2M3 digit table (above)
 __device__ inline void write_q8_lane(int q, uint16_t dh, int lane, size_t blk, int8_t *codes,
                                      float *scales, uint8_t *mxtab, uint8_t *blocks34,
-                                     uint32_t *btab = nullptr) {
+                                     uint8_t *dtab = nullptr) {
     if (lane >= 32) return;
-    if (btab)
-        reinterpret_cast<uint16_t *>(btab + blk * 16)[2 * (lane & 15) + (lane >> 4)] =
-            (uint16_t)(__float_as_uint((float)q) >> 16);
+    if (dtab) {
+        // lanes 0-15 pack the h digits, 16-31 the l digits: elements i and
+        // i + 16 side by side (12 bits at lane i), then a quad's 48 bits,
+        // stored as three 16-bit words by its first three lanes
+        const uint32_t own = e2m3_small(q >> 4) | (uint32_t)(q & 15) << 8;
+        const uint32_t oth = (uint32_t)__builtin_amdgcn_ds_swizzle((int)own, 0x401F);  // lane ^ 16
+        const bool lo = lane >= 16;
+        const uint32_t p12 = lo ? (oth >> 8 | (own >> 8) << 6) : ((own & 63u) | (oth & 63u) << 6);
+        const uint32_t x = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p12, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+        const uint32_t p24 = (lane & 1) ? (x | p12 << 12) : (p12 | x << 12);
+        const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p24, 0x4E, 0xF, 0xF, false);  // lane ^ 2
+        const int c = lane & 3;
+        const uint32_t A = c < 2 ? p24 : y, B = c < 2 ? y : p24;
+        const uint32_t w = c == 0 ? A : c == 1 ? (A >> 16 | B << 8) : B >> 8;
+        uint8_t *t = dtab + blk * kDigitBytes;
+        if (c < 3) *reinterpret_cast<uint16_t *>(t + digit_byte(lo, 6 * ((lane & 15) >> 2) + 2 * c)) = (uint16_t)w;
+        else if ((lane & 15) == 3) *reinterpret_cast<float *>(t + digit_scale(lo)) = f16_bits_to_f32(dh);
+    }
     if (codes) codes[blk * 32 + lane] = (int8_t)q;
     if (scales && lane == 0) scales[blk] = f16_bits_to_f32(dh);
     if (mxtab) {
@@ -500,6 +494,52 @@ __device__ inline float swiglu(float gate, float up) {
     u = (u < -7.0f) ? -7.0f : u;
     float e = static_cast<float>(exp_f64<KREG>(static_cast<double>(-1.702f * g)));
     return g / (1.0f + e) * (u + 1.0f);
+}
+
+// N SwiGLU values at once: the same operations, the exp's constants taken
+// once (scalar registers) for all of them.
+template <int N>
+__device__ __attribute__((always_inline)) inline void swiglu_n(const float (&gate)[N], const float (&up)[N], float (&out)[N]) {
+    constexpr int KREG = kConstSgpr;
+    float g[N], u[N];
+    double k[N], r[N], p[N];
+    const double l2e = SPT_KD(1.4426950408889634), ln2l = SPT_KD(1.90821492927058770002e-10),
+                 ln2h = SPT_KD(6.93147180369123816490e-01);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        g[i] = (gate[i] > 7.0f) ? 7.0f : gate[i];
+        u[i] = (up[i] > 7.0f) ? 7.0f : up[i];
+        u[i] = (u[i] < -7.0f) ? -7.0f : u[i];
+        // x >= -11.92 (or NaN, where the quotient is NaN whatever the exp);
+        // beyond 100 the exp is Inf as a float, as at 100
+        const double x = static_cast<double>(fminf(-1.702f * g[i], 100.0f));
+        k[i] = __builtin_rint(x * l2e);
+        r[i] = __builtin_fma(-k[i], ln2l, __builtin_fma(-k[i], ln2h, x));
+        p[i] = 1.0 / 87178291200.0;  // 1/14!
+    }
+    auto step = [&](double c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < N; i++) p[i] = __builtin_fma(p[i], r[i], c);
+    };
+    step(SPT_KD(1.0 / 6227020800.0));
+    step(SPT_KD(1.0 / 479001600.0));
+    step(SPT_KD(1.0 / 39916800.0));
+    step(SPT_KD(1.0 / 3628800.0));
+    step(SPT_KD(1.0 / 362880.0));
+    step(SPT_KD(1.0 / 40320.0));
+    step(SPT_KD(1.0 / 5040.0));
+    step(SPT_KD(1.0 / 720.0));
+    step(SPT_KD(1.0 / 120.0));
+    step(SPT_KD(1.0 / 24.0));
+    step(SPT_KD(1.0 / 6.0));
+    step(0.5);
+    step(1.0);
+    step(1.0);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const double e = __builtin_ldexp(p[i], (int)k[i]);
+        out[i] = g[i] / (1.0f + static_cast<float>(e)) * (u[i] + 1.0f);
+    }
 }
 
 }  // namespace spt

@@ -10,11 +10,14 @@ namespace spt {
 
 constexpr int kMaxTopK = 16;
 constexpr int kMaxExperts = 256;
-constexpr int kMaxSelections = 4096;
+constexpr int kMaxSelections = 4096;   // per call with taps or without allocation
+constexpr int kSliceSelections = 8192;  // per launch sequence of the other calls
 // Tokens of an expert's list per pass of the grouped GEMV over its weights.
 constexpr int kGemvTokens = 4;
-// List entries per work item of the grouped GEMM (spt_mx_gemm.hip).
+// List entries per pass of the grouped wide product (spt_mx_wide.hip), and
+// the output rows of its units.
 constexpr int kGemmTokens = 64;
+constexpr int kWideRows = 32;
 // Largest MXFP4 input dimension of the grouped GEMV: a workgroup stages four
 // 16-row tiles of whole rows in LDS (GPT-OSS uses 2880 for both projections).
 constexpr int kMxMaxInput = 2880;
@@ -27,21 +30,29 @@ struct SelectOut {
     int32_t *list;
     int32_t *active;
     int32_t *n_active;
-    // Experts with count >= gemm_min go to the grouped GEMM, the others to
+    // Experts with count >= gemm_min go to the wide launches, the others to
     // the grouped GEMV, each with its own packed expert list:
     int32_t gemm_min;
-    // ...provided their GEMM work items (token tiles x gemm_units row units)
-    // number at least gemm_min_items (enough to fill the device); otherwise
-    // every expert goes to the GEMV.
-    int32_t gemm_units;
-    int32_t gemm_min_items;
+    // ...provided they gain at least gemm_min_gain over the GEMV's passes (in
+    // the units of wide_cost and kGemvPassCost) and hold at least gemm_min_units
+    // units (passes x wide_units[0]: enough to fill the device); otherwise every
+    // expert goes to the GEMV.
+    int32_t gemm_min_gain, gemm_min_units;
+    // With fewer than gv_min_experts experts below gemm_min, those go to the
+    // wide launches too.
+    int32_t gv_min_experts;
     int32_t *gv_active;    // [E] GEMV experts, ascending
     int32_t *gv_n;
     int32_t *gv_pass_off;  // [E+1] prefix over GEMV experts of ceil(count / kGemvTokens)
-    int32_t *gm_active;    // [E] GEMM experts, by descending count (equal counts ascending)
-    int32_t *gm_n;
-    int32_t *gm_tile_off;  // [E+1] prefix over GEMM experts of ceil(count / kGemmTokens)
-    int32_t *gm_claim;     // [2] work-item counters of the two GEMM launches (zeroed)
+    int32_t *gm_active;    // [E] experts of the wide launches, by descending count (equal counts ascending)
+    // Work of the two wide launches (gate/up, down) for gm_grid workgroups:
+    // for workgroup b of launch l, kGvStartWords ints at
+    // gm_start[(l * kGvStartMax + b) * kGvStartWords]: its number of units; the
+    // slot, pass and unit of the first (wide_units[l] units per pass); that
+    // slot's expert, list begin and count.
+    int32_t *gm_start;
+    int32_t gm_grid;
+    int32_t wide_units[2];
     // Optional start table of the two grouped GEMV launches (gate/up, down):
     // for workgroup b of launch l, kGvStartWords ints at
     // gv_start[(l * kGvStartMax + b) * kGvStartWords]: its item range
@@ -51,7 +62,7 @@ struct SelectOut {
     int32_t gv_grid[2];
     int32_t gv_tiles[2];
 };
-constexpr int kGvStartMax = 1024;
+constexpr int kGvStartMax = 512;
 constexpr int kGvStartWords = 8;
 
 // Optional Q8_0 outputs of a quantized activation (see write_q8_block);
@@ -62,7 +73,7 @@ struct QuantOut {
     float *scales;
     uint8_t *mxtab;
     uint8_t *blocks34;
-    uint32_t *btab;
+    uint8_t *dtab;
     const uint8_t *src34;
 };
 
@@ -129,36 +140,32 @@ struct DecDownArgs {
 hipError_t launch_dec_gate_up(hipStream_t s, const DecGateUpArgs &a, int n_sel);
 hipError_t launch_dec_down(hipStream_t s, const DecDownArgs &a, int batch);
 
-// Grouped MXFP4 x Q8_0 GEMM on the bf16 MFMA (spt_mx_gemm.hip) for the
-// experts of the GEMM list (SelectOut.gm_*): the kGateUp and kDown
-// semantics of MxMfmaArgs, with the activations read as bf16 code tables
-// (write_q8_block's btab layout) and the gate/up epilogue also writing the
-// btab table of act.
-struct MxGemmArgs {
+// Grouped MXFP4 x Q8_0 product of up to kGemmTokens list entries per pass
+// (spt_mx_wide.hip) for the experts of SelectOut::gm_active: the
+// kGateUp and kDown semantics of MxMfmaArgs, with the activations read as
+// E2M3 digit tables (write_q8_lane's dtab layout) and the gate/up epilogue
+// writing that table of act.
+struct MxWideArgs {
     const uint8_t *w[2];
     uint64_t expert_bytes;
-    int rows;
+    int rows;                // a multiple of kWideRows
     int nb;
-    const void *bias[2];
+    const void *bias[2];     // aligned to their elements
+    uint64_t bias_bytes[2];
     int bias_type[2];
-    const uint32_t *btab;    // activation bf16 code tables [tab_rows][nb][16 dwords]
-    int64_t tab_rows;        // rows of btab, scales and codes
-    const float *scales;     // activation Q8_0 scales [*][nb]
+    const uint8_t *tab;      // activation digit tables [*][nb][kDigitBytes]
+    uint32_t tab_bytes;
     const int8_t *codes;     // activation Q8_0 codes [*][nb*32] (special-scale rows)
-    const int32_t *gm_active;
-    const int32_t *gm_n;
-    const int32_t *gm_tile_off;
-    int32_t *claim;          // work-item counter, zero at launch (items past the first G are claimed)
+    const int32_t *active;   // SelectOut::gm_active
+    const int32_t *start;    // this launch's rows of SelectOut::gm_start
     const int32_t *offsets;
     const int32_t *list;
     int topk;
     float *out;
     float *tap[2];
     int8_t *act_codes;
-    float *act_scales;
-    uint8_t *act_mxtab;
+    uint8_t *act_tab;
     uint8_t *act_blocks34;
-    uint32_t *act_btab;
 };
 
 // One more Q4_0 matrix of a GEMV launch over several projections of the
@@ -258,7 +265,7 @@ struct Q80Args {
 
 hipError_t launch_quantize(hipStream_t s, const float *x, int64_t nblocks, int8_t *codes,
                            float *scales, int32_t *sumq, uint8_t *mxtab, uint8_t *blocks34,
-                           uint32_t *btab);
+                           uint8_t *dtab);
 // Router logits [batch][experts]; Q8_0 of x into q when q.codes or q.blocks34 is set.
 hipError_t launch_route(hipStream_t s, const float *router, const void *bias, int bias_type,
                         const float *x, int batch, int hidden, int experts, float *logits,
@@ -276,8 +283,12 @@ int device_cus();
 hipError_t launch_mx_mfma(hipStream_t s, GemvMode mode, const MxMfmaArgs &a, int slots);
 // The grid launch_mx_mfma uses for these arguments (0: nothing to launch).
 int mx_mfma_grid(GemvMode mode, const MxMfmaArgs &a, int slots);
-// max_items: upper bound of the GEMM work items (0: nothing to launch).
-hipError_t launch_mx_gemm(hipStream_t s, GemvMode mode, const MxGemmArgs &a, int max_items);
+// The grid of launch_mx_wide (SelectOut::gm_grid).
+int mx_wide_grid();
+// Whether the wide launches take expert matrices of this many bytes (their
+// loads use offsets past 2^31 for "nothing").
+inline bool mx_wide_fits(uint64_t expert_bytes) { return expert_bytes <= 0x7FFFFF00ull; }
+hipError_t launch_mx_wide(hipStream_t s, GemvMode mode, const MxWideArgs &a);
 // Q4_0 x Q8_0 for a batch: the int8-MFMA GEMM (spt_q40_gemm.hip, tiles of
 // kQ40TileRows rows x kQ40TileTokens tokens) from kQ40GemmMinTokens tokens
 // on kQ40GemmMinRows output rows and more, and from kQ40SplitMinTokens

@@ -7,6 +7,7 @@
 // of the workgroup's tokens) are staged in LDS once and shared by the rows.
 // The MXFP4 GEMV lives in spt_mx_mfma.hip.
 #include <atomic>
+#include <climits>
 
 #include "spt_device.h"
 #include "spt_kernels.h"
@@ -27,14 +28,14 @@ __global__ __launch_bounds__(kWG) void k_quantize(const float *__restrict__ x, i
                                                   int32_t *__restrict__ sumq,
                                                   uint8_t *__restrict__ mxtab,
                                                   uint8_t *__restrict__ blocks34,
-                                                  uint32_t *__restrict__ btab) {
+                                                  uint8_t *__restrict__ dtab) {
     const int tid = threadIdx.x, lane = tid & 63, i = tid & 31;
     const int64_t b = (int64_t)blockIdx.x * (kWG / 32) + (tid >> 5);
     const bool ok = b < nblocks;
     const float v = ok ? x[b * 32 + i] : 0.0f;
     uint16_t dh;
     const int q = q8_quantize_half(v, lane, &dh);  // every lane takes part (cross-lane steps)
-    if (ok) write_q8_lane(q, dh, i, (size_t)b, codes, scales, mxtab, blocks34, btab);
+    if (ok) write_q8_lane(q, dh, i, (size_t)b, codes, scales, mxtab, blocks34, dtab);
     if (sumq) {
         int s = q;
 #pragma unroll
@@ -45,10 +46,10 @@ __global__ __launch_bounds__(kWG) void k_quantize(const float *__restrict__ x, i
 
 hipError_t launch_quantize(hipStream_t s, const float *x, int64_t nblocks, int8_t *codes,
                            float *scales, int32_t *sumq, uint8_t *mxtab, uint8_t *blocks34,
-                           uint32_t *btab) {
+                           uint8_t *dtab) {
     if (nblocks <= 0) return hipSuccess;
     dim3 grid((unsigned)((nblocks + kWG / 32 - 1) / (kWG / 32)));
-    hipLaunchKernelGGL(k_quantize, grid, dim3(kWG), 0, s, x, nblocks, codes, scales, sumq, mxtab, blocks34, btab);
+    hipLaunchKernelGGL(k_quantize, grid, dim3(kWG), 0, s, x, nblocks, codes, scales, sumq, mxtab, blocks34, dtab);
     return hipGetLastError();
 }
 
@@ -121,47 +122,93 @@ __device__ __attribute__((always_inline)) inline int lane63(int x) { return __bu
 // held in LDS (s_ids/s_w), by one workgroup of kSelWG threads.  Selections
 // with Weight <= 0 are skipped (NaN weights are kept); experts ascending;
 // inside a list descending idx, as the reference's push-at-head linked list
-// yields.  Counts by LDS atomics, offsets and the active-expert list by one
-// wavefront's prefix scan; ranks from kSelChunk-entry chunks taken in
-// descending idx order: a per-expert bit row marks the chunk's members, so an
-// entry's rank is its expert's running count plus the bits below it.
+// yields.  Each of the sixteen wavefronts takes a contiguous part of the
+// selections in descending idx order: per wavefront and expert counts by LDS
+// atomics, offsets and the active-expert list by one wavefront's prefix scan,
+// then every wavefront places its part 64 entries at a time, an entry's rank
+// among the lanes of its expert by ballots over the expert's bits (4096
+// selections: 25.8 us with one chunk of 512 at a time between barriers).
 constexpr int kSelWG = 1024;
-static_assert(kSelWG >= 4 * kMaxExperts, "four threads per expert rank the GEMM experts");
-constexpr int kSelChunk = 512;
-constexpr int kSelWords = kSelChunk / 32;
+static_assert(kSelWG >= 4 * kMaxExperts, "four threads per expert rank the wide launches' experts");
+constexpr int kSelWaves = kSelWG / 64;
+constexpr int kExpertBits = 8;
+static_assert(kMaxExperts <= 1 << kExpertBits, "expert ids");
+
+// Cost of a unit of a wide pass with one and with two 32-entry tiles, of a
+// unit of all passes over a list of c entries, and of the same rows in a GEMV
+// pass: tenths of a microsecond per expert on the whole device, gate/up at
+// GPT-OSS-120B shape (2.5, 3.7; GEMV 1.4).
+constexpr int kWideCost1 = 25, kWideCost2 = 37, kGemvPassCost = 14;
+__device__ inline int wide_cost(int c) {
+    const int full = c / kGemmTokens, rem = c % kGemmTokens;
+    return full * kWideCost2 + (rem == 0 ? 0 : rem > 32 ? kWideCost2 : kWideCost1);
+}
+
+// Last i < n with v[i] <= x, v ascending and v[0] <= x (0 for n = 0).
+__device__ inline int last_at_most(const int32_t *v, int n, int x) {
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (v[mid] <= x) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
 
 __device__ void pack_lists(int n, int E, const SelectOut &o, const int32_t *s_ids, const float *s_w,
-                           int32_t *s_cnt, int32_t *s_off, int32_t *s_run, uint32_t *s_bits) {
-    __shared__ int s_gemm_on, s_nv;
+                           int32_t *s_cnt, int32_t *s_off, int32_t *s_wcnt) {
+    __shared__ int s_gemm_min, s_nv, s_nm, s_ntile, s_cost;
     // the GEMV experts and their pass prefix, for the start table
-    int32_t *s_poff = reinterpret_cast<int32_t *>(s_bits + kSelWords * E);
+    int32_t *s_poff = s_wcnt + kSelWaves * E;
     int32_t *s_gva = s_poff + E + 1;
+    // the wide launches' experts' pass and cost prefixes, for theirs
+    int32_t *s_gmt = s_gva + E;
+    int32_t *s_gmc = s_gmt + E + 1;
     const int tid = threadIdx.x;
-    for (int i = tid; i < E; i += blockDim.x) {
-        s_cnt[i] = 0;
-        s_run[i] = 0;
+    const int wave = tid >> 6, lane = tid & 63;
+    // this wavefront's selections: places [p0, p1) in descending idx order
+    // (of whole wavefronts of entries: fewer selections, fewer parts)
+    const int per = max(64, (n + kSelWaves - 1) / kSelWaves), parts = (n + per - 1) / per;
+    const int p0 = min(wave * per, n), p1 = min(p0 + per, n);
+    for (int i = tid; i < parts * E; i += blockDim.x) s_wcnt[i] = 0;
+    __syncthreads();
+    for (int p = p0 + lane; p < p1; p += 64) {
+        const int idx = n - 1 - p;
+        if (!(s_w[idx] <= 0.0f)) atomicAdd(&s_wcnt[wave * E + s_ids[idx]], 1);
     }
     __syncthreads();
-    for (int i = tid; i < n; i += blockDim.x)
-        if (!(s_w[i] <= 0.0f)) atomicAdd(&s_cnt[s_ids[i]], 1);
+    // the wavefronts' counts -> their places inside each expert's list
+    for (int e = tid; e < E; e += blockDim.x) {
+        int run = 0;
+        for (int w = 0; w < parts; w++) {
+            const int c = s_wcnt[w * E + e];
+            s_wcnt[w * E + e] = run;
+            run += c;
+        }
+        s_cnt[e] = run;
+    }
     __syncthreads();
     if (tid < 64) {
         // offsets (scan of counts), the active list, and the GEMV expert
         // list with its prefix (passes of kGemvTokens) in ascending expert
-        // order; the GEMM experts' count and tiles (ordered below)
+        // order; the number of the wide launches' experts and passes (ordered below)
         int pos = 0, na = 0, nv = 0, nm = 0, npass = 0, ntile = 0;
         const uint64_t below = (1ull << tid) - 1ull;
-        // GEMM work items the threshold would give
-        int tiles = 0;
+        // what the wide passes over the threshold's experts would save, and the
+        // experts below it
+        int gain = 0, small = 0, passes = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int c = e0 + tid < E ? s_cnt[e0 + tid] : 0;
-            tiles += lane63(wave_incl_scan((c > 0 && c >= o.gemm_min) ? (c + kGemmTokens - 1) / kGemmTokens : 0));
+            small += __builtin_popcountll(__ballot(c > 0 && c < o.gemm_min));
+            gain += lane63(wave_incl_scan((c > 0 && c >= o.gemm_min) ? (c + kGemvTokens - 1) / kGemvTokens * kGemvPassCost - wide_cost(c) : 0));
+            passes += lane63(wave_incl_scan((c > 0 && c >= o.gemm_min) ? (c + kGemmTokens - 1) / kGemmTokens : 0));
         }
-        const bool gemm_on = (int64_t)tiles * o.gemm_units >= (int64_t)o.gemm_min_items;
+        const bool gemm_on = gain >= o.gemm_min_gain && (int64_t)passes * o.wide_units[0] >= o.gemm_min_units;
+        const int gm_min = gemm_on && small < o.gv_min_experts ? 1 : o.gemm_min;
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int e = e0 + tid;
             const int c = e < E ? s_cnt[e] : 0;
-            const bool big = gemm_on && c > 0 && c >= o.gemm_min;
+            const bool big = gemm_on && c > 0 && c >= gm_min;
             const int np = big ? 0 : (c + kGemvTokens - 1) / kGemvTokens;
             const int ntl = big ? (c + kGemmTokens - 1) / kGemmTokens : 0;
             const int incl = wave_incl_scan(c), pincl = wave_incl_scan(np), tincl = wave_incl_scan(ntl);
@@ -194,40 +241,76 @@ __device__ void pack_lists(int n, int E, const SelectOut &o, const int32_t *s_id
             o.gv_pass_off[nv] = npass;
             s_poff[nv] = npass;
             s_nv = nv;
-            *o.gm_n = nm;
-            o.gm_tile_off[nm] = ntile;
-            if (o.gm_claim) {
-                o.gm_claim[0] = 0;
-                o.gm_claim[1] = 0;
-            }
-            s_gemm_on = gemm_on;
+            s_nm = nm;
+            s_ntile = ntile;
+            s_gemm_min = gemm_on ? gm_min : INT_MAX;
         }
     }
-    // The GEMM experts by descending count (equal counts by ascending id), so
-    // the GEMM's work items, claimed in order by workgroups as they free up,
-    // end with the smallest: an expert's rank and tile prefix count the GEMM
-    // experts ordered before it.
-    // Four threads per expert, each counting over a quarter of the experts
-    // (kSelWG >= 4 * kMaxExperts), summed across the four lanes.
+    // The wide launches' experts by descending count (equal counts by ascending id):
+    // an expert's rank, pass prefix and cost prefix count those ordered
+    // before it.  Four threads per expert, each counting over a
+    // quarter of the experts (kSelWG >= 4 * kMaxExperts), summed across the
+    // four lanes.
+    if (tid == 0) s_cost = 0;
     __syncthreads();
-    if (s_gemm_on && tid < 4 * E) {
+    const int gemm_min = s_gemm_min;
+    if (gemm_min < INT_MAX && tid < 4 * E) {
         const int e = tid >> 2, part = tid & 3, q = (E + 3) / 4;
         const int c = s_cnt[e];
-        int rank = 0, pre = 0;
+        int rank = 0, pre = 0, cost = 0;
         for (int f = part * q; f < min(E, part * q + q); f++) {
             const int cf = s_cnt[f];
-            if (cf > 0 && cf >= o.gemm_min && (cf > c || (cf == c && f < e))) {
+            if (cf > 0 && cf >= gemm_min && (cf > c || (cf == c && f < e))) {
                 rank++;
                 pre += (cf + kGemmTokens - 1) / kGemmTokens;
+                cost += wide_cost(cf);
             }
         }
         rank += __shfl_xor(rank, 1);
         pre += __shfl_xor(pre, 1);
+        cost += __shfl_xor(cost, 1);
         rank += __shfl_xor(rank, 2);
         pre += __shfl_xor(pre, 2);
-        if (part == 0 && c > 0 && c >= o.gemm_min) {
+        cost += __shfl_xor(cost, 2);
+        if (part == 0 && c > 0 && c >= gemm_min) {
             o.gm_active[rank] = e;
-            o.gm_tile_off[rank] = pre;
+            s_gmt[rank] = pre;
+            s_gmc[rank] = cost;
+            atomicAdd(&s_cost, wide_cost(c));
+        }
+    }
+    __syncthreads();
+    // Start table of the two wide launches: workgroup b of G takes the units
+    // whose cost positions lie in [b W / G, (b + 1) W / G) of the whole.
+    if (o.gm_start) {
+        const int nm = s_nm, ntile = s_ntile;
+        for (int i = tid; i < 2 * o.gm_grid; i += blockDim.x) {
+            const int l = i >= o.gm_grid, b = i - l * o.gm_grid, units = o.wide_units[l];
+            const int64_t W = nm > 0 ? (int64_t)s_cost * units : 0;
+            int ord[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int64_t x = (int64_t)(b + k) * W / o.gm_grid;
+                // the slot holding position x, then the pass and the unit at or above it
+                const int lo = last_at_most(s_gmc, nm, (int)(units > 0 ? x / units : 0));
+                if (nm == 0 || x >= W) {
+                    ord[k] = ntile * units;
+                    continue;
+                }
+                const int c = s_cnt[o.gm_active[lo]];
+                const int64_t r = x - (int64_t)s_gmc[lo] * units;
+                const int full = c / kGemmTokens;
+                const int p = min((int)(r / ((int64_t)kWideCost2 * units)), c % kGemmTokens ? full : full - 1);
+                const int cp = min(c - p * kGemmTokens, kGemmTokens) > 32 ? kWideCost2 : kWideCost1;
+                const int64_t in = r - (int64_t)p * kWideCost2 * units;
+                ord[k] = (s_gmt[lo] + p) * units + (int)((in + cp - 1) / cp);
+            }
+            const int t = units > 0 ? ord[0] / units : 0;
+            const int lo = last_at_most(s_gmt, nm, t);
+            const int e = nm > 0 ? o.gm_active[lo] : 0;
+            int32_t *d = o.gm_start + ((size_t)l * kGvStartMax + b) * kGvStartWords;
+            *reinterpret_cast<int4 *>(d) = make_int4(ord[1] - ord[0], lo, nm > 0 ? t - s_gmt[lo] : 0, units > 0 ? ord[0] % units : 0);
+            *reinterpret_cast<int4 *>(d + 4) = make_int4(e, s_off[e], s_cnt[e], 0);
         }
     }
     // Start table of the two GEMV launches (threads [0, G0) the first,
@@ -244,46 +327,38 @@ __device__ void pack_lists(int n, int E, const SelectOut &o, const int32_t *s_id
             const int W = P * tiles;
             const int w0 = (int)((int64_t)b * W / G), w1 = (int)((int64_t)(b + 1) * W / G);
             const int q0 = tiles > 0 ? w0 / tiles : 0;
-            int lo = 0, hi = nv - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (s_poff[mid] <= q0) lo = mid;
-                else hi = mid - 1;
-            }
+            const int lo = last_at_most(s_poff, nv, q0);
             int32_t *d = o.gv_start + ((size_t)l * kGvStartMax + b) * kGvStartWords;
             *reinterpret_cast<int4 *>(d) = make_int4(w0, w1, lo, nv > 0 ? s_gva[lo] : 0);
             d[4] = nv > 0 ? q0 - s_poff[lo] : 0;
         }
     }
-    for (int p0 = 0; p0 < n; p0 += kSelChunk) {
-        for (int i = tid; i < E * kSelWords; i += blockDim.x) s_bits[i] = 0u;
-        __syncthreads();
-        const int p = p0 + tid;
-        const int idx = n - 1 - p;
-        const bool valid = tid < kSelChunk && p < n && !(s_w[idx] <= 0.0f);
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (int q = p0; q < p1; q += 64) {
+        const int p = q + lane, idx = n - 1 - p;
+        const bool valid = p < p1 && !(s_w[idx] <= 0.0f);
         const int e = valid ? s_ids[idx] : 0;
-        if (valid) atomicOr(&s_bits[e * kSelWords + (tid >> 5)], 1u << (tid & 31));
-        __syncthreads();
+        uint64_t same = __ballot(valid);  // the valid lanes of this lane's expert
+#pragma unroll
+        for (int b = 0; b < kExpertBits; b++) {
+            const bool bit = (e >> b) & 1;
+            const uint64_t m = __ballot(bit);
+            same &= bit ? m : ~m;
+        }
+        // (one wavefront's LDS operations complete in order)
+        volatile int32_t *run = &s_wcnt[wave * E + e];
+        const int base = *run, rank = __builtin_popcountll(same & below);
         if (valid) {
-            int rank = s_run[e];
-            const int wi = tid >> 5;
-            for (int w = 0; w < wi; w++) rank += __builtin_popcount(s_bits[e * kSelWords + w]);
-            rank += __builtin_popcount(s_bits[e * kSelWords + wi] & ((1u << (tid & 31)) - 1u));
-            o.list[s_off[e] + rank] = idx;
+            o.list[s_off[e] + base + rank] = idx;
+            if (rank == 0) *run = base + __builtin_popcountll(same);
         }
-        __syncthreads();
-        for (int i = tid; i < E; i += blockDim.x) {
-            int add = 0;
-            for (int w = 0; w < kSelWords; w++) add += __builtin_popcount(s_bits[i * kSelWords + w]);
-            s_run[i] += add;
-        }
-        __syncthreads();
     }
 }
 
+// ids and weights, counts, offsets, the wavefronts' counts, and the prefixes
+// of the start tables
 static size_t select_lds(int n, int E) {
-    return sizeof(int32_t) * (2 * (size_t)n + 3 * (size_t)E + 1) + sizeof(uint32_t) * kSelWords * (size_t)E +
-           sizeof(int32_t) * (2 * (size_t)E + 1);
+    return sizeof(int32_t) * (2 * (size_t)n + 2 * (size_t)E + 1 + kSelWaves * (size_t)E + 4 * (size_t)E + 2);
 }
 
 // Router logits for batches of more than kRouteLdsMaxBatch tokens: a
@@ -320,7 +395,7 @@ __global__ __launch_bounds__(kWG) void k_route_tile(const float *__restrict__ ro
                 const float v = f < nq ? x[(size_t)t * H + b * 32 + i] : 0.0f;
                 qv = q8_quantize_half(v, lane, &dh);  // every lane takes part
             }
-            if (f < nq) write_q8_lane(qv, dh, i, (size_t)t * nbh + b, q.codes, q.scales, q.mxtab, q.blocks34, q.btab);
+            if (f < nq) write_q8_lane(qv, dh, i, (size_t)t * nbh + b, q.codes, q.scales, q.mxtab, q.blocks34, q.dtab);
         }
     }
     const int e0 = blockIdx.x * 4 + EW * (wave % (4 / EW)), t0 = tg0 + TT * (wave / (4 / EW));
@@ -431,7 +506,7 @@ __global__ __launch_bounds__(64) void k_route(const float *__restrict__ router, 
         if (s0 == 0 && qon) {
             uint16_t dh = qdh;
             const int qv = q.src34 ? qcode : q8_quantize_half(qin, lane, &dh);  // every lane takes part
-            if (qb < nbh) write_q8_lane(qv, dh, qi, (size_t)t * nbh + qb, q.codes, q.scales, q.mxtab, q.blocks34, q.btab);
+            if (qb < nbh) write_q8_lane(qv, dh, qi, (size_t)t * nbh + qb, q.codes, q.scales, q.mxtab, q.blocks34, q.dtab);
         }
         __syncthreads();  // the previous segment's LDS reads are done
 #pragma unroll
@@ -460,8 +535,7 @@ __global__ __launch_bounds__(kSelWG) void k_select(const float *__restrict__ log
     float *s_w = reinterpret_cast<float *>(smem_i + n);
     int32_t *s_cnt = smem_i + 2 * n;
     int32_t *s_off = s_cnt + E;
-    int32_t *s_run = s_off + E + 1;
-    uint32_t *s_bits = reinterpret_cast<uint32_t *>(s_run + E);
+    int32_t *s_wcnt = s_off + E + 1;
     const int wave = threadIdx.x >> 6;
     // each wave takes tokens wave, wave + 16, ...; the next token's logits
     // are loaded while the current one is selected
@@ -474,7 +548,7 @@ __global__ __launch_bounds__(kSelWG) void k_select(const float *__restrict__ log
         select_token(cur, E, topk, o.ids + t * topk, o.weights + t * topk, s_ids + t * topk, s_w + t * topk);
     }
     __syncthreads();
-    pack_lists(n, E, o, s_ids, s_w, s_cnt, s_off, s_run, s_bits);
+    pack_lists(n, E, o, s_ids, s_w, s_cnt, s_off, s_wcnt);
 }
 
 // Large batches: the selections first, a wavefront per token over the whole
@@ -497,14 +571,13 @@ __global__ __launch_bounds__(kSelWG) void k_pack(int batch, int E, int topk, Sel
     float *s_w = reinterpret_cast<float *>(smem_i + n);
     int32_t *s_cnt = smem_i + 2 * n;
     int32_t *s_off = s_cnt + E;
-    int32_t *s_run = s_off + E + 1;
-    uint32_t *s_bits = reinterpret_cast<uint32_t *>(s_run + E);
+    int32_t *s_wcnt = s_off + E + 1;
     for (int i = threadIdx.x; i < n; i += kSelWG) {
         s_ids[i] = o.ids[i];
         s_w[i] = o.weights[i];
     }
     __syncthreads();
-    pack_lists(n, E, o, s_ids, s_w, s_cnt, s_off, s_run, s_bits);
+    pack_lists(n, E, o, s_ids, s_w, s_cnt, s_off, s_wcnt);
 }
 
 int device_cus() {
@@ -567,6 +640,11 @@ hipError_t launch_route(hipStream_t s, const float *router, const void *bias, in
 }
 
 hipError_t launch_pack(hipStream_t s, int batch, int experts, int topk, const SelectOut &o) {
+    // one-time opt-in to more than 64 KB of dynamic LDS
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pack), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)select_lds(kSliceSelections, kMaxExperts));
+    if (attr != hipSuccess) return attr;
+    if (batch * topk > kSliceSelections) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_pack, dim3(1), dim3(kSelWG), select_lds(batch * topk, experts), s, batch, experts, topk, o);
     return hipGetLastError();
 }
@@ -584,8 +662,7 @@ hipError_t launch_select(hipStream_t s, const float *logits, int batch, int expe
                        experts, topk, o.ids, o.weights);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pack, dim3(1), dim3(kSelWG), select_lds(batch * topk, experts), s, batch, experts, topk, o);
-    return hipGetLastError();
+    return launch_pack(s, batch, experts, topk, o);
 }
 
 // ---------------------------------------------------------------------------
