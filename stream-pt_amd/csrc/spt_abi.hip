@@ -988,7 +988,7 @@ int run_q40_at(spt_ctx *ctx, const Q40Proj *p, int np, const Q40Plan &L, char *S
     if (L.views) {
         SPT_HIP(timed(ctx, SPT_KERNEL_QUANTIZE, [&] {
             return x ? spt::launch_quantize(ctx->stream, x, batch * nb, codes, scales, sumq, nullptr, nullptr, nullptr)
-                     : spt::launch_q8_unpack(ctx->stream, xq34, batch * nb, codes, scales, sumq, nullptr);
+                     : spt::launch_q8_unpack(ctx->stream, xq34, batch * nb, codes, scales, sumq);
         }));
     }
     // the three launches' arguments: 0 GEMV, 1 wide GEMM, 2 split GEMM

@@ -294,8 +294,11 @@ hipError_t launch_mx_wide(hipStream_t s, GemvMode mode, const MxWideArgs &a);
 // on kQ40GemmMinRows output rows and more, and from kQ40SplitMinTokens
 // tokens on narrower projections; else the GEMV.  The GEMM splits K
 // kQ40SplitK ways (partial sums in Q40Args::part, then summed in order,
-// when the caller provides the scratch) for narrow projections and for wide
-// ones of fewer than kQ40SplitMaxTiles tiles (too few to fill the device).
+// when the caller provides the scratch) for projections of fewer than
+// kQ40SplitMaxTiles tiles (too few to fill the device); wider or longer ones
+// run unsplit, in the same launch as the others of their call (K and V of
+// 512 rows at 1,999 tokens: 55 us split and 12 us of reduction beside Q's 154,
+// against 40 more in Q's launch).
 // Unsplit, its sums are the GEMV's bit for bit; split, the partial sums of
 // the K ranges are added in range order (within rounding of the GEMV).
 constexpr int kQ40TileRows = 64;
@@ -310,9 +313,8 @@ inline bool q40_gemm_form(int64_t rows, int64_t ntok) {
            (ntok >= kQ40SplitMinTokens && rows < kQ40GemmMinRows);
 }
 inline bool q40_gemm_split(int64_t rows, int64_t ntok) {
-    return rows < kQ40GemmMinRows ||
-           ((rows + kQ40TileRows - 1) / kQ40TileRows) * ((ntok + kQ40TileTokens - 1) / kQ40TileTokens) <
-               kQ40SplitMaxTiles;
+    return ((rows + kQ40TileRows - 1) / kQ40TileRows) * ((ntok + kQ40TileTokens - 1) / kQ40TileTokens) <
+           kQ40SplitMaxTiles;
 }
 // The GEMV stages its tokens' activations (40 bytes per block) in at most
 // kQ40GemvLds bytes of LDS, at least one token per pass: inputs up to
@@ -332,7 +334,7 @@ hipError_t launch_q40_dec(hipStream_t s, const Q40Args &a);
 // GGML Q8_0 blocks -> codes, widened scales and per-block code sums (the
 // views launch_quantize writes), for nblocks blocks.
 hipError_t launch_q8_unpack(hipStream_t s, const uint8_t *blocks34, int64_t nblocks, int8_t *codes,
-                            float *scales, int32_t *sumq, uint8_t *mxtab);
+                            float *scales, int32_t *sumq);
 hipError_t launch_q40_gemm(hipStream_t s, const Q40Args &a);
 // 5 to 64 tokens of inputs up to 128 blocks (spt_q40_tile.hip): a
 // workgroup per 16 output rows (when those workgroups all fit on the n_cu

@@ -462,3 +462,45 @@ def test_mxfp4_expert_unaligned_base(gpu_ctx, O, off, batch):
         outs.append(y.cpu().numpy())
         del buf
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("batch", [32, 65, 131])
+def test_q40_views_of_fp32_and_blocks(gpu_ctx, O, batch):
+    """The GEMM's activation views (k_q40_views) from fp32 rows and from their
+    GGML Q8_0 blocks give the same bits, with the rows 4 bytes and the blocks
+    2 bytes past a 16-byte boundary, ragged token tiles, and blocks of zeros,
+    subnormals, halves (codes at .5), infinities and NaN among them."""
+    import torch
+
+    from spt import synth
+
+    din, dout = 1056, 1100
+    import spt
+
+    w = synth.q40_bytes(synth.stream_key(8, dout), dout, din)
+    wd = torch.from_numpy(w).cuda()
+    t = spt.Tensor.make("attn_output", spt.TYPE_Q4_0, [din, dout], wd.data_ptr(), w.size)
+    x = synth.normal(synth.stream_key(41, batch), batch * din).reshape(batch, din).copy()
+    x[1, :32] = 0.0
+    x[2, 32:64] = np.float32(1e-44)
+    x[3, :32] = np.arange(32, dtype=np.float32) + np.float32(0.5)
+    x[3, 31] = 127.0
+    x[4, 64] = np.inf
+    x[5, 96] = np.nan
+    xd = torch.zeros(batch * din + 1, dtype=torch.float32, device="cuda")[1:]
+    xd.copy_(torch.from_numpy(x.reshape(-1)))
+    q = torch.zeros(batch * din // 32 * 34 + 2, dtype=torch.uint8, device="cuda")[2:]
+    gpu_ctx.quantize_q8_0(xd, q)
+    a = torch.zeros(batch * dout, dtype=torch.float32, device="cuda")
+    b = torch.zeros(batch * dout, dtype=torch.float32, device="cuda")
+    gpu_ctx.mul_q40_batch_into(t, xd, a, batch)
+    gpu_ctx.mul_q40_qkv_batch_into([t, t, t], None, None, [b, torch.zeros_like(b), torch.zeros_like(b)], batch, xq=q,
+                                   x_len=batch * din)
+    torch.cuda.synchronize()
+    ah, bh = a.cpu().numpy().reshape(batch, dout), b.cpu().numpy().reshape(batch, dout)
+    assert np.array_equal(np.isnan(ah), np.isnan(bh)) and np.isnan(ah[5]).all()
+    ok = ~np.isnan(ah)
+    assert np.array_equal(ah[ok].view(np.uint32), bh[ok].view(np.uint32))
+    rows = [r for r in range(batch) if r not in (4, 5)]
+    want = O.mul_q40_q8(w, np.ascontiguousarray(x[rows]).reshape(-1), din, dout, len(rows))
+    assert_close(ah[rows].reshape(-1), want, what="Q4_0 from fp32")
