@@ -162,6 +162,10 @@ hipError_t timed(spt_ctx *ctx, int kind, F &&launch) {
 }
 
 // Grow-only device scratch arena; returns a pointer to at least `bytes` bytes.
+// The first allocation is large enough that a context's first few calls (the
+// projections of a layer, then its experts) do not each grow it: growing
+// waits for the stream and costs about 0.5 ms.
+constexpr size_t kArenaMin = size_t(32) << 20;
 int arena(spt_ctx *ctx, size_t bytes, char **out) {
     if (bytes > ctx->scratch_bytes) {
         if (ctx->scratch) {
@@ -171,7 +175,7 @@ int arena(spt_ctx *ctx, size_t bytes, char **out) {
             ctx->scratch = nullptr;
             ctx->scratch_bytes = 0;
         }
-        size_t want = bytes + bytes / 4 + 4096;
+        const size_t want = std::max(bytes + bytes / 4 + 4096, kArenaMin);
         if (hipMalloc(&ctx->scratch, want) != hipSuccess) {
             ctx->scratch = nullptr;
             return fail(SPT_ERR_NOMEM, "cannot allocate %zu bytes of device scratch", want);
@@ -914,7 +918,7 @@ void q40_launches(const Q40Proj *p, int np, int64_t batch, int *k) {
 // runs as one launch over every projection reading GGML Q8_0 blocks: the
 // caller's, or those the quantizer writes into the arena (o_q34) first.
 struct Q40Plan {
-    bool views, dec, tile;
+    bool views, dec, tile, gemm;
     int64_t nb, batch;
     size_t o_c, o_s, o_q, o_part, o_q34, total;
 };
@@ -935,6 +939,7 @@ Q40Plan q40_plan(const Q40Proj *p, int np, int64_t nb, int64_t batch, bool q8_in
         if (k[i] == 2) part += (size_t)spt::kQ40SplitK * batch * p[i].out * 4;
     }
     L.views = !L.dec && !L.tile && (!q8_in || gemm);
+    L.gemm = gemm;
     L.nb = nb;
     L.batch = batch;
     Carve c;
@@ -987,8 +992,7 @@ int run_q40_at(spt_ctx *ctx, const Q40Proj *p, int np, const Q40Plan &L, char *S
     int32_t *sumq = L.views ? (int32_t *)(S + L.o_q) : nullptr;
     if (L.views) {
         SPT_HIP(timed(ctx, SPT_KERNEL_QUANTIZE, [&] {
-            return x ? spt::launch_quantize(ctx->stream, x, batch * nb, codes, scales, sumq, nullptr, nullptr, nullptr)
-                     : spt::launch_q8_unpack(ctx->stream, xq34, batch * nb, codes, scales, sumq);
+            return spt::launch_q40_views(ctx->stream, x, xq34, batch * nb, L.gemm, codes, scales, sumq);
         }));
     }
     // the three launches' arguments: 0 GEMV, 1 wide GEMM, 2 split GEMM

@@ -316,6 +316,10 @@ inline bool q40_gemm_split(int64_t rows, int64_t ntok) {
     return ((rows + kQ40TileRows - 1) / kQ40TileRows) * ((ntok + kQ40TileTokens - 1) / kQ40TileTokens) <
            kQ40SplitMaxTiles;
 }
+// Place of code dword i (elements 4i .. 4i + 3) of a block in the views of a
+// batch in GEMM form: dwords g and g + 4, the K elements of lane group g of
+// the MFMA, side by side.  Smaller batches' views keep the order.
+__host__ __device__ inline int q40_code_dword(int i) { return 2 * (i & 3) + (i >> 2); }
 // The GEMV stages its tokens' activations (40 bytes per block) in at most
 // kQ40GemvLds bytes of LDS, at least one token per pass: inputs up to
 // kQ40MaxInput elements.
@@ -331,10 +335,11 @@ constexpr int kQ40DecMaxNb = 128;
 constexpr uint64_t kQ40DecMaxBytes = 0x80000000ull;
 inline bool q40_dec_form(int64_t batch, int64_t nb) { return batch <= kQ40DecTokens && nb <= kQ40DecMaxNb; }
 hipError_t launch_q40_dec(hipStream_t s, const Q40Args &a);
-// GGML Q8_0 blocks -> codes, widened scales and per-block code sums (the
-// views launch_quantize writes), for nblocks blocks.
-hipError_t launch_q8_unpack(hipStream_t s, const uint8_t *blocks34, int64_t nblocks, int8_t *codes,
-                            float *scales, int32_t *sumq);
+// The views of Q4_0 calls: codes (with `gemm` in the order of q40_code_dword),
+// widened scales and per-block code sums, for nblocks blocks of fp32 (x) or
+// GGML Q8_0 (blocks34) input.
+hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, bool gemm,
+                            int8_t *codes, float *scales, int32_t *sumq);
 hipError_t launch_q40_gemm(hipStream_t s, const Q40Args &a);
 // 5 to 64 tokens of inputs up to 128 blocks (spt_q40_tile.hip): a
 // workgroup per 16 output rows (when those workgroups all fit on the n_cu

@@ -66,7 +66,7 @@ __device__ __attribute__((always_inline)) inline uint32_t max8_bits(uint32_t m) 
 // q8_quantize_half's.  Memory-bound: 8.2 M elements, 42 MB, from fp32 25.6 us
 // with a lane per element, from blocks (5.8 M, 12 MB) 15.0 us.
 template <bool Q8>
-__global__ __launch_bounds__(kWG) void k_q40_views(const void *__restrict__ in, int64_t nblocks,
+__global__ __launch_bounds__(kWG) void k_q40_views(const void *__restrict__ in, int64_t nblocks, bool gemm,
                                                    int8_t *__restrict__ codes, float *__restrict__ scales,
                                                    int32_t *__restrict__ sumq) {
     const int tid = threadIdx.x, lane = tid & 63, i = tid & 7;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kWG) void k_q40_views(const void *__restrict__ in, 
     }
     const int s = sum8_int(__builtin_amdgcn_sdot4((int)w, 0x01010101, 0, false));
     if (!ok) return;
-    reinterpret_cast<uint32_t *>(codes)[b * 8 + i] = w;
+    reinterpret_cast<uint32_t *>(codes)[b * 8 + (gemm ? q40_code_dword(i) : i)] = w;
     if (i == 0) {
         scales[b] = f16_bits_to_f32(dh);
         sumq[b] = s;
@@ -111,21 +111,19 @@ hipError_t launch_quantize(hipStream_t s, const float *x, int64_t nblocks, int8_
                            float *scales, int32_t *sumq, uint8_t *mxtab, uint8_t *blocks34,
                            uint8_t *dtab) {
     if (nblocks <= 0) return hipSuccess;
-    if (codes && scales && sumq && !mxtab && !blocks34 && !dtab) {
-        hipLaunchKernelGGL(k_q40_views<false>, dim3((unsigned)((nblocks + kWG / 8 - 1) / (kWG / 8))), dim3(kWG), 0, s, x, nblocks, codes,
-                           scales, sumq);
-        return hipGetLastError();
-    }
     dim3 grid((unsigned)((nblocks + kWG / 32 - 1) / (kWG / 32)));
     hipLaunchKernelGGL(k_quantize, grid, dim3(kWG), 0, s, x, nblocks, codes, scales, sumq, mxtab, blocks34, dtab);
     return hipGetLastError();
 }
 
-hipError_t launch_q8_unpack(hipStream_t s, const uint8_t *blocks34, int64_t nblocks, int8_t *codes,
-                            float *scales, int32_t *sumq) {
+hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, bool gemm,
+                            int8_t *codes, float *scales, int32_t *sumq) {
     if (nblocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_q40_views<true>, dim3((unsigned)((nblocks + kWG / 8 - 1) / (kWG / 8))), dim3(kWG), 0, s, blocks34, nblocks,
-                       codes, scales, sumq);
+    const dim3 grid((unsigned)((nblocks + kWG / 8 - 1) / (kWG / 8)));
+    if (x)
+        hipLaunchKernelGGL(k_q40_views<false>, grid, dim3(kWG), 0, s, x, nblocks, gemm, codes, scales, sumq);
+    else
+        hipLaunchKernelGGL(k_q40_views<true>, grid, dim3(kWG), 0, s, blocks34, nblocks, gemm, codes, scales, sumq);
     return hipGetLastError();
 }
 
@@ -870,14 +868,6 @@ hipError_t launch_q40_gemv(hipStream_t s, const Q40Args &a) {
         if (per_lane <= 4) return launch_q40_maxp<4>(s, a);
         if (per_lane <= 6) return launch_q40_maxp<6>(s, a);
         return launch_q40_maxp<8>(s, a);
-    }
-    if (q40_gemm_form(a.rows, a.ntok)) {
-        // split K with the caller's scratch where the form asks for it;
-        // without scratch, wide projections take the GEMM unsplit and
-        // narrow ones the GEMV
-        Q40Args g = a;
-        if (!q40_gemm_split(a.rows, a.ntok)) g.part = nullptr;
-        if (g.part || a.rows >= kQ40GemmMinRows) return launch_q40_gemm(s, g);
     }
     const int per_lane = (a.nb + 15) / 16;
     if (per_lane <= 1) return launch_q40_maxp<1>(s, a);

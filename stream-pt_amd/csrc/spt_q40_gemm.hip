@@ -10,7 +10,13 @@
 // GEMV's arithmetic per block.
 // K order inside a block: lane group g of the MFMA (k = 8g .. 8g+7) takes
 // nibble bytes 2+4g .. 5+4g of the block: low nibbles are elements 4g..4g+3,
-// high nibbles 16+4g..16+4g+3, matched by code dwords g and 4+g.
+// high nibbles 16+4g..16+4g+3, matched by code dwords g and 4+g, which the
+// views hold side by side (q40_code_dword), one 8-byte LDS read.
+// What bounds it: LDS reads beside three VALU operations per output and
+// block.  A block of a wave (16 rows x 64 tokens) takes seven LDS reads: its
+// nibbles, four rows' d_w, the fragments' d_x, and four 8-byte code reads
+// (seventeen with scales and code dwords read one by one: Q and O at 1,999
+// tokens 150 and 152 us then).
 // MFMA lane layout (measured on the hardware): lane l holds A row l%16 and
 // B column l%16 at k = 8*(l/16) + 0..7 (byte i of the 64-bit operand is
 // k offset i); D lane l, register r is row 4*(l/16) + r, column l%16.
@@ -41,8 +47,9 @@ constexpr int kBSlots = 2 * kSeg + 1;        // LDS slots of 16 B per staged tok
 constexpr int kBTok = 16 * kBSlots;          // 68 dwords: a fragment's tokens over distinct banks
 constexpr int kBInstr = kTN * kBSlots / 64;  // LDS DMA loads of a stage's B: 17
 constexpr int kOffB = kTR * kARow;
-constexpr int kOffD = kOffB + kTN * kBTok;  // d_x [kSeg][token] (a fragment's 16 tokens in consecutive banks)
+constexpr int kOffD = kOffB + kTN * kBTok;  // d_x [kSeg][entry i16 of a fragment][fragment]
 constexpr int kStageBytes = kOffD + kTN * kSeg * 4;
+constexpr int kDwBytes = 16 * kSeg * 4;      // a wave's d_w of a segment as f32 [kSeg][row], after the stages
 constexpr uint32_t kOOR = 0x80000000u;      // buffer offset past every range: reads zero
 static_assert(kSeg * kQ40Block + 15 <= 16 * kAPieces && kAPieces < kASlots, "A window");
 static_assert(kTR * kASlots % 64 == 0, "whole A loads");
@@ -63,7 +70,8 @@ __device__ __attribute__((always_inline)) inline uint32_t word_at(const uint8_t 
 // of its MFMAs.
 struct Q40Lane {
     uint32_t alead;     // LDS offset of this lane's nibble word of block 0
-    uint32_t dlead[4];  // LDS offsets of the D rows' fp16 scales of block 0
+    uint32_t slead;     // LDS offset of its row's fp16 scale of block 0
+    float *dw;          // the wave's d_w [kSeg][16]
     int i16, g;
 };
 
@@ -72,40 +80,40 @@ __device__ __attribute__((always_inline)) inline void q40_blocks(const uint8_t *
                                                                  float (&acc)[4][4]) {
     struct Blk {
         uint32_t w4;
-        uint32_t dwb[4];
-        uint32_t bq[NTF][2];
-        float dx[NTF];
+        v4f dw;
+        uint2 bq[NTF];
+        v4f dx;
     };
     auto fetch = [&](int j, Blk &b) {
         b.w4 = word_at(st, L.alead + (uint32_t)j * kQ40Block);
+        b.dw = *reinterpret_cast<const v4f *>(L.dw + 16 * j + 4 * L.g);
+        b.dx = *reinterpret_cast<const v4f *>(st + kOffD + 4 * j * kTN + 16 * L.i16);
 #pragma unroll
-        for (int r = 0; r < 4; r++) b.dwb[r] = *reinterpret_cast<const uint16_t *>(st + L.dlead[r] + (uint32_t)j * kQ40Block);
-#pragma unroll
-        for (int tf = 0; tf < NTF; tf++) {
-            const int t = 16 * tf + L.i16;
-            const uint32_t *bq = reinterpret_cast<const uint32_t *>(st + kOffB + t * kBTok + 32 * j);
-            b.bq[tf][0] = bq[L.g];
-            b.bq[tf][1] = bq[4 + L.g];
-            b.dx[tf] = *reinterpret_cast<const float *>(st + kOffD + 4 * (j * kTN + t));
-        }
+        for (int tf = 0; tf < NTF; tf++)
+            b.bq[tf] = *reinterpret_cast<const uint2 *>(st + kOffB + (16 * tf + L.i16) * kBTok + 32 * j + 8 * L.g);
     };
     auto run = [&](const Blk &b) {
         // per byte: nibble n -> n - 8 as int8
         const uint32_t lo = (((b.w4 & 0x0F0F0F0Fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
         const uint32_t hi = ((((b.w4 >> 4) & 0x0F0F0F0Fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
         const long A = (long)lo | ((long)hi << 32);
-        float dw[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) dw[r] = f16_bits_to_f32(b.dwb[r]);
         v4i D[NTF];
 #pragma unroll
         for (int tf = 0; tf < NTF; tf++)
-            D[tf] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, (long)b.bq[tf][0] | ((long)b.bq[tf][1] << 32), v4i{0, 0, 0, 0}, 0, 0, 0);
+            D[tf] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, (long)b.bq[tf].x | ((long)b.bq[tf].y << 32), v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
         for (int tf = 0; tf < NTF; tf++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) acc[tf][r] = __builtin_fmaf((float)D[tf][r], dw[r] * b.dx[tf], acc[tf][r]);
+            for (int r = 0; r < 4; r++) acc[tf][r] = __builtin_fmaf((float)D[tf][r], b.dw[r] * b.dx[tf], acc[tf][r]);
     };
+    // The wave's 16 x kSeg weight scales once per segment, widened, so that a
+    // block reads its four D rows' by one 16-byte load (a lane: row i16, blocks
+    // g and g + 4; a wave's LDS operations complete in order).
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+        L.dw[16 * (L.g + 4 * h) + L.i16] = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(st + L.slead + (uint32_t)(L.g + 4 * h) * kQ40Block));
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
     if constexpr (JN > 0) {
         Blk cur, nxt;
         fetch(0, cur);
@@ -204,20 +212,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
         for (int k = 0; k < kDLoads; k++) {
             const int b = b0 + wave + kWaves * k;
-            const uint32_t off = (lane < nt && b < kb1) ? ((uint32_t)(t0 + lane) * (uint32_t)nb + (uint32_t)b) * 4u : kOOR;
+            // lane 4 * i16 + tf: fragment tf's entry i16, so a lane's four fragments' d_x are one 16-byte read
+            const int t = 16 * (lane & 3) + (lane >> 2);
+            const uint32_t off = (t < nt && b < kb1) ? ((uint32_t)(t0 + t) * (uint32_t)nb + (uint32_t)b) * 4u : kOOR;
             dma4(rsd, st + kOffD + 256u * (uint32_t)(wave + kWaves * k), off, 0u);
         }
     };
 
-    // this lane's A row (MFMA layout: row i16) and D rows (4g .. 4g+3)
+    // this lane's A row (MFMA layout: row i16)
     const int arow = 16 * wave + i16;
     const uint32_t apos = le + (uint32_t)(r0 + arow < a.rows ? r0 + arow : 0) * row_bytes;
-    uint32_t dpos[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int row = r0 + 16 * wave + 4 * g + r;
-        dpos[r] = le + (uint32_t)(row < a.rows ? row : 0) * row_bytes;
-    }
     float acc[4][4];
 #pragma unroll
     for (int tf = 0; tf < 4; tf++)
@@ -230,14 +234,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     auto kloop = [&](auto ntf_c) {
         constexpr int NTF = decltype(ntf_c)::value;
         auto lane_of = [&](int s) {
-            // window offsets of segment s: A row (nibble bytes 2+4g..5+4g of
-            // block j at lead + 18j + 2 + 4g), and the D rows' scales
+            // window offsets of segment s: the A row's scale, and its nibble
+            // bytes 2+4g..5+4g of block j at lead + 18j + 2 + 4g
             const int b0 = kb0 + s * kSeg;
             Q40Lane L;
-            L.alead = (uint32_t)arow * kARow + ((apos + (uint32_t)b0 * kQ40Block) & 15u) + 2u + 4u * (uint32_t)g;
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-                L.dlead[r] = (uint32_t)(16 * wave + 4 * g + r) * kARow + ((dpos[r] + (uint32_t)b0 * kQ40Block) & 15u);
+            L.slead = (uint32_t)arow * kARow + ((apos + (uint32_t)b0 * kQ40Block) & 15u);
+            L.alead = L.slead + 2u + 4u * (uint32_t)g;
+            L.dw = reinterpret_cast<float *>(lds + 2 * kStageBytes + wave * kDwBytes);
             L.i16 = i16;
             L.g = g;
             return L;
@@ -338,7 +341,7 @@ hipError_t launch_q40_gemm(hipStream_t s, const Q40Args &a) {
     }
     const int ks = a.part ? (a.nb < kQ40SplitK ? a.nb : kQ40SplitK) : 1;
     dim3 grid(tiles, (a.ntok + kTN - 1) / kTN, ks);
-    hipLaunchKernelGGL(k_q40_gemm, grid, dim3(kThreads), 2 * (size_t)kStageBytes, s, a);
+    hipLaunchKernelGGL(k_q40_gemm, grid, dim3(kThreads), 2 * (size_t)kStageBytes + kWaves * kDwBytes, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !a.part) return e;
     const size_t n = (size_t)a.ntok * rows;
