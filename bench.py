@@ -35,7 +35,7 @@ HBM_PEAK_GBPS = 8000.0
 BF16_DENSE_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
 INT8_DENSE_TOPS = 5000.0     # MI355X dense int8 MFMA
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_mx_mfma_decode_b64_36layers.md")
-MFMA_PROFILE = os.path.join(ROOT, "profiles", "k_mx_gemm_prefill_b512_hot.md")
+MFMA_PROFILE = os.path.join(ROOT, "profiles", "k_mx_wide_prefill_b512_hot.md")
 # policy of the library's default for the wide launches (spt_abi.hip:
 # kGemmMinGroup, kGemmMinSelections, kGemmMinGain, kGemvMinExperts;
 # spt_kernels.hip: the costs of a wide pass of one and of two tiles and of a
@@ -431,8 +431,8 @@ def prefill(args, ctx, dl, shp, W, stream, reps=20):
         if gemm_sel and gemm_us > 0:
             macs = gemm_sel * 3 * H * D
             tops = 2 * macs / (gemm_us * 1e-6) / 1e12
-            res["gemm"] = {"mfma": "bf16 (v_mfma_f32_16x16x32_bf16)", "macs": macs, "us": round(gemm_us, 1),
-                           "tflops_bf16": round(tops, 2), "frac_bf16_dense": round(tops / BF16_DENSE_TFLOPS, 4),
+            res["gemm"] = {"mfma": "FP4 x FP6 (v_mfma_scale_f32_32x32x64_f8f6f4, two digits a code)", "macs": macs, "us": round(gemm_us, 1),
+                           "tflops": round(tops, 2), "frac_bf16_dense": round(tops / BF16_DENSE_TFLOPS, 4),
                            "mfma_util_measured": measured_mfma_util(name)}
         if name == "hot_b512":
             qa = q40_projections(ctx, B, W, stream, reps)

@@ -407,6 +407,53 @@ static size_t select_lds(int n, int E) {
     return sizeof(int32_t) * (2 * (size_t)n + 2 * (size_t)E + 1 + kSelWaves * (size_t)E + 4 * (size_t)E + 2);
 }
 
+// The Q8_0 of `tokens` rows of x from tg0 on (or their unpacking from q.src34),
+// shared by the workgroups of a row of the grid: a half-wave per block.
+__device__ __attribute__((always_inline)) inline void route_quantize(const float *__restrict__ x, int tg0, int tokens, int H,
+                                                                     const QuantOut &q) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (!q.codes && !q.blocks34) return;
+    // four blocks' inputs in flight at once: with one, a half-wave's loads and
+    // stores took longer than the logits of large batches
+    constexpr int kBatch = 4;
+    const int nbh = H / 32, nq = tokens * nbh, i = tid & 31, step = gridDim.x * (kWG / 32);
+    for (int f0 = blockIdx.x * (kWG / 32); f0 < nq; f0 += kBatch * step) {
+        float v[kBatch];
+        int qv[kBatch];
+        uint16_t dh[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; k++) {
+            const int f = f0 + k * step + (tid >> 5), fi = f < nq ? f : 0;
+            const size_t blk = (size_t)tg0 * nbh + fi;
+            if (q.src34) {
+                const uint8_t *b = q.src34 + blk * kQ80Block;
+                qv[k] = (int)(int8_t)b[2 + i];
+                dh[k] = (uint16_t)(b[0] | (b[1] << 8));
+            } else {
+                v[k] = x[blk * 32 + i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; k++) {
+            const int f = f0 + k * step + (tid >> 5);
+            if (!q.src34) qv[k] = q8_quantize_half(f < nq ? v[k] : 0.0f, lane, &dh[k]);  // every lane takes part
+            if (f < nq) write_q8_lane(qv[k], dh[k], i, (size_t)tg0 * nbh + f, q.codes, q.scales, q.mxtab, q.blocks34, q.dtab);
+        }
+    }
+}
+
+// This lane's value plus that of the lane 16 (32) away.
+__device__ __attribute__((always_inline)) inline float sum_permlane16(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+__device__ __attribute__((always_inline)) inline float sum_permlane32(float v) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+
 // Router logits for batches of more than kRouteLdsMaxBatch tokens: a
 // workgroup per (4 experts, EW * TT tokens), its four wavefronts in a
 // (4 / EW) x EW arrangement of (EW experts, TT tokens) each.  Lane L keeps one
@@ -425,25 +472,7 @@ __global__ __launch_bounds__(kWG) void k_route_tile(const float *__restrict__ ro
     constexpr int TW = EW * TT;  // tokens per workgroup (U: chunks per pass of loads)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tg0 = blockIdx.y * TW;
-    if (q.codes || q.blocks34) {
-        const int nbh = H / 32, nq = min(TW, B - tg0) * nbh;
-        for (int f0 = blockIdx.x * (kWG / 32); f0 < nq; f0 += gridDim.x * (kWG / 32)) {
-            const int f = f0 + (tid >> 5), i = tid & 31;
-            const int fi = f < nq ? f : 0;
-            const int t = tg0 + fi / nbh, b = fi % nbh;
-            uint16_t dh;
-            int qv;
-            if (q.src34) {
-                const uint8_t *blk = q.src34 + ((size_t)t * nbh + b) * kQ80Block;
-                qv = (int)(int8_t)blk[2 + i];
-                dh = (uint16_t)(blk[0] | (blk[1] << 8));
-            } else {
-                const float v = f < nq ? x[(size_t)t * H + b * 32 + i] : 0.0f;
-                qv = q8_quantize_half(v, lane, &dh);  // every lane takes part
-            }
-            if (f < nq) write_q8_lane(qv, dh, i, (size_t)t * nbh + b, q.codes, q.scales, q.mxtab, q.blocks34, q.dtab);
-        }
-    }
+    route_quantize(x, tg0, min(TW, B - tg0), H, q);
     const int e0 = blockIdx.x * 4 + EW * (wave % (4 / EW)), t0 = tg0 + TT * (wave / (4 / EW));
     if (e0 >= E || t0 >= B) return;  // whole wavefronts
     const float *wr[EW], *xr[TT];
@@ -494,6 +523,91 @@ __global__ __launch_bounds__(kWG) void k_route_tile(const float *__restrict__ ro
             if (lane == 0 && e0 + i < E && t0 + j < B)
                 logits[(size_t)(t0 + j) * E + e0 + i] = r + bias_at(bias, bias_type, e0 + i);
         }
+}
+
+// The same for large batches: a workgroup per (16 experts, 16 tokens), its
+// four wavefronts of (8 experts, 8 tokens) each.  A wavefront's rows are read
+// whole from the caches, 16 rows for 64 logits (half the bytes of the 4 x 4
+// tile, which bound it), U chunks of every row in flight; the lanes' partial
+// sums go through LDS sixteen logits at a time, where four lanes add up a
+// logit's in the order of router_reduce (seven shuffles a logit there).  Same
+// bits.
+template <int U>
+__global__ __launch_bounds__(kWG) void k_route_wide(const float *__restrict__ router, const void *bias,
+                                                    int bias_type, const float *__restrict__ x, int B, int H, int E,
+                                                    float *__restrict__ logits, QuantOut q) {
+    constexpr int EW = 8, TT = 8, kPitch = 68;
+    __shared__ float s_part[kWG / 64][16 * kPitch];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tg0 = blockIdx.y * 2 * TT;
+    route_quantize(x, tg0, min(2 * TT, B - tg0), H, q);
+    const int e0 = blockIdx.x * 2 * EW + EW * (wave & 1), t0 = tg0 + TT * (wave >> 1);
+    if (e0 >= E || t0 >= B) return;  // whole wavefronts
+    const float *wr[EW], *xr[TT];
+#pragma unroll
+    for (int i = 0; i < EW; i++) wr[i] = router + (size_t)min(e0 + i, E - 1) * H;
+#pragma unroll
+    for (int j = 0; j < TT; j++) xr[j] = x + (size_t)min(t0 + j, B - 1) * H;
+    float acc[EW][TT];
+#pragma unroll
+    for (int i = 0; i < EW; i++)
+#pragma unroll
+        for (int j = 0; j < TT; j++) acc[i][j] = 0.0f;
+    // as in k_route_tile: chunks past the row load its last chunk and are not
+    // multiplied
+    const int nfull = H / 64;
+    for (int c0 = 0; c0 < nfull; c0 += U) {
+        float wv[U][EW], xv[U][TT];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int c = min(c0 + u, nfull - 1) * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < EW; i++) wv[u][i] = wr[i][c];
+#pragma unroll
+            for (int j = 0; j < TT; j++) xv[u][j] = xr[j][c];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (c0 + u < nfull) {
+#pragma unroll
+                for (int i = 0; i < EW; i++)
+#pragma unroll
+                    for (int j = 0; j < TT; j++) acc[i][j] = __builtin_fmaf(wv[u][i], xv[u][j], acc[i][j]);
+            }
+        }
+    }
+    if (nfull * 64 < H && lane < 32) {
+#pragma unroll
+        for (int i = 0; i < EW; i++)
+#pragma unroll
+            for (int j = 0; j < TT; j++)
+                acc[i][j] = __builtin_fmaf(wr[i][nfull * 64 + lane], xr[j][nfull * 64 + lane], acc[i][j]);
+    }
+    // logits of tokens 2b, 2b + 1: lane L (logit n = L % 16, part p = L / 16)
+    // adds up AVX2 accumulators p and p + 4 of the eight
+    float *sp = s_part[wave];
+    const int n = lane & 15, p = lane >> 4;
+#pragma unroll
+    for (int b = 0; b < TT / 2; b++) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) sp[k * kPitch + lane] = acc[k & 7][2 * b + (k >> 3)];
+        // (one wavefront's LDS operations complete in order)
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+        float a[2][8];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int k = 0; k < 8; k++) a[h][k] = sp[n * kPitch + 8 * k + p + 4 * h];
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        float t[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) t[h] = (((a[h][0] + a[h][1]) + a[h][2]) + a[h][3]) + (((a[h][4] + a[h][5]) + a[h][6]) + a[h][7]);
+        const float r = sum_permlane32(sum_permlane16(t[0] + t[1]));
+        const int e = e0 + (n & 7), tok = t0 + 2 * b + (n >> 3);
+        if (p == 0 && e < E && tok < B) logits[(size_t)tok * E + e] = r + bias_at(bias, bias_type, e);
+    }
 }
 
 // Router logits: one wavefront per (expert, token), a workgroup each, so a
@@ -656,7 +770,14 @@ hipError_t launch_route(hipStream_t s, const float *router, const void *bias, in
         // CUs, in passes of 23 chunks (76 VGPRs; measured while this form
         // also took 8 tokens: 7.1-7.5 against 7.9 us there, and 9.6-9.9
         // against 10.7-12.6 at 31, with one pass of 45).
-        if (batch >= 256) {
+        // (8 x 8 wavefronts of k_route_wide from 384 workgroups of 16 x 16, six
+        // wavefronts a compute unit; 128 experts, us, 4 x 4 / 8 x 8: 512 tokens
+        // 38 / 43, 768: 47 / 47, 1000: 61 / 47, 2000: 108 / 64)
+        const dim3 wide((experts + 15) / 16, (batch + 15) / 16);
+        if (wide.x * wide.y >= 384) {
+            hipLaunchKernelGGL(k_route_wide<3>, wide, dim3(kWG), 0, s, router, bias, bias_type, x, batch, hidden, experts,
+                               logits, q);
+        } else if (batch >= 256) {
             dim3 grid((experts + 3) / 4, (batch + 15) / 16);
             hipLaunchKernelGGL((k_route_tile<4, 4, 15>), grid, dim3(kWG), 0, s, router, bias, bias_type, x, batch,
                                hidden, experts, logits, q);

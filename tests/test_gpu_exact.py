@@ -135,7 +135,7 @@ def exact_layer():
 def test_moe_kernels_exact(gpu_ctx, O, exact_layer, path, batch):
     """Decode kernels (k_dec_gate_up / k_dec_down: up to 8 selections on the
     default path, 12 when forced), the grouped GEMV (k_mx_mfma kGateUp / kDown) and the
-    grouped GEMM (k_mx_gemm, every group forced onto it): the gate and up
+    grouped GEMM (k_mx_wide, every group forced onto it): the gate and up
     taps equal the integer form over the full 2,880-input rows, every
     selection's down result the single rounding of its one block, and the
     usual stage-wise checks hold (ids, packing, SwiGLU, act Q8_0, combine)."""

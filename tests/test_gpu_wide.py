@@ -85,3 +85,28 @@ def test_pack_lists_order(gpu_ctx, O, batch, topk, experts):
     counts, offsets, lst, active = O.group(g["ids"], g["weights"], batch, topk, experts)
     assert np.array_equal(g["counts"], counts) and np.array_equal(g["offsets"], offsets)
     assert np.array_equal(g["list"][:offsets[-1]], lst)
+
+
+@pytest.mark.parametrize("hidden,experts,batch", [(2880, 128, 771), (96, 37, 2053), (4128, 256, 385)])
+def test_route_wide_bits(gpu_ctx, O, hidden, experts, batch):
+    """The large-batch router (8 x 8 logits a wavefront, 384 workgroups and
+    more) gives the reference's accumulation order bit for bit: ragged experts
+    and tokens, and a trailing half chunk of 32 elements."""
+    import torch
+
+    import spt
+
+    rng = np.random.default_rng(hidden + batch)
+    w = rng.standard_normal((experts, hidden)).astype(np.float32)
+    b = rng.standard_normal(experts).astype(np.float32)
+    x = rng.standard_normal((batch, hidden)).astype(np.float32)
+    wd, bd, xd = (torch.from_numpy(v).cuda() for v in (w, b, x))
+    t = spt.Tensor.make("ffn_gate_inp.weight", spt.TYPE_F32, [hidden, experts], wd.data_ptr(), w.nbytes)
+    tb = spt.Tensor.make("ffn_gate_inp.bias", spt.TYPE_F32, [experts], bd.data_ptr(), b.nbytes)
+    out = torch.empty(batch * experts, dtype=torch.float32, device="cuda")
+    gpu_ctx.route_moe_batch(t, tb, xd, batch, out)
+    torch.cuda.synchronize()
+    rows = sorted({0, 1, 7, 8, 15, 16, batch // 2, batch - 2, batch - 1})
+    want = O.route(w.reshape(-1), b, np.ascontiguousarray(x[rows]).reshape(-1), len(rows), hidden, experts)
+    got = out.cpu().numpy().reshape(batch, experts)[rows]
+    assert np.array_equal(bits(got.reshape(-1)), bits(np.asarray(want, np.float32).reshape(-1)))
