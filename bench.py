@@ -353,8 +353,8 @@ def prefill(args, ctx, dl, shp, W, stream, reps=20):
     the library's stream), the weight bytes of the touched experts over the
     layer time, and for the grouped GEMM its algorithmic multiply-adds
     (selections of GEMM experts x 3 x hidden x expert dim) over its kernel
-    time against the dense bf16 MFMA peak it runs on (it issues bf16 MFMAs
-    only); at 512 tokens, the Q4_0 projections' int8 MFMA rate (the int8
+    time against the dense bf16 MFMA peak (its FP4 x FP6 MFMAs multiply each
+    code as two digits); at 512 tokens, the Q4_0 projections' int8 MFMA rate (the int8
     MFMA kernel of this path) against the dense int8 peak."""
     import numpy as np
     import torch

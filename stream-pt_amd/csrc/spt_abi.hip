@@ -162,11 +162,8 @@ hipError_t timed(spt_ctx *ctx, int kind, F &&launch) {
 }
 
 // Grow-only device scratch arena; returns a pointer to at least `bytes` bytes.
-// The first allocation is large enough that a context's first few calls (the
-// projections of a layer, then its experts) do not each grow it: growing
-// waits for the stream and costs about 0.5 ms.
-constexpr size_t kArenaMin = size_t(32) << 20;
-int arena(spt_ctx *ctx, size_t bytes, char **out) {
+// `more`: what the layer's next call is likely to ask for on top.
+int arena(spt_ctx *ctx, size_t bytes, char **out, size_t more = 0) {
     if (bytes > ctx->scratch_bytes) {
         if (ctx->scratch) {
             hipError_t e = hipStreamSynchronize(ctx->stream);
@@ -175,7 +172,7 @@ int arena(spt_ctx *ctx, size_t bytes, char **out) {
             ctx->scratch = nullptr;
             ctx->scratch_bytes = 0;
         }
-        const size_t want = std::max(bytes + bytes / 4 + 4096, kArenaMin);
+        const size_t want = bytes + std::max(bytes / 4, more) + 4096;
         if (hipMalloc(&ctx->scratch, want) != hipSuccess) {
             ctx->scratch = nullptr;
             return fail(SPT_ERR_NOMEM, "cannot allocate %zu bytes of device scratch", want);
@@ -921,6 +918,12 @@ struct Q40Plan {
     bool views, dec, tile, gemm;
     int64_t nb, batch;
     size_t o_c, o_s, o_q, o_part, o_q34, total;
+    // A GEMM batch leaves room for its size again, up to 16 MB: O follows Q/K/V
+    // with an input that is often wider, and growing the arena waits for the
+    // stream and costs about 0.5 ms (740 us instead of 160 for such a layer's
+    // first pass). Smaller batches gain nothing: there the larger allocation
+    // alone was 45 us of a first pass of 90.
+    size_t room() const { return gemm ? std::min(total, size_t(16) << 20) : 0; }
 };
 
 Q40Plan q40_plan(const Q40Proj *p, int np, int64_t nb, int64_t batch, bool q8_in, size_t base) {
@@ -1357,7 +1360,7 @@ int spt_mul_q40_batch_bias_into(spt_ctx *ctx, const spt_tensor *w, const spt_ten
     p.resid = resid_dev;
     const Q40Plan plan = q40_plan(&p, 1, in / 32, batch, false, 0);
     char *S;
-    if ((rc = arena(ctx, plan.total, &S))) return rc;
+    if ((rc = arena(ctx, plan.total, &S, plan.room()))) return rc;
     return run_q40_at(ctx, &p, 1, plan, S, x_dev, nullptr);
 }
 
@@ -1376,7 +1379,7 @@ int spt_mul_q40_batch_q8_into(spt_ctx *ctx, const spt_tensor *w, const spt_tenso
     p.resid = resid_dev;
     const Q40Plan plan = q40_plan(&p, 1, in / 32, batch, true, 0);
     char *S;
-    if ((rc = arena(ctx, plan.total, &S))) return rc;
+    if ((rc = arena(ctx, plan.total, &S, plan.room()))) return rc;
     return run_q40_at(ctx, &p, 1, plan, S, nullptr, (const uint8_t *)xq_dev);
 }
 
@@ -1417,7 +1420,7 @@ int spt_mul_q40_qkv_batch_into(spt_ctx *ctx, const spt_tensor *w, const spt_tens
     if ((rc = check_device(ctx))) return rc;
     const Q40Plan plan = q40_plan(p, 3, in / 32, batch, xq_dev != nullptr, 0);
     char *S;
-    if ((rc = arena(ctx, plan.total, &S))) return rc;
+    if ((rc = arena(ctx, plan.total, &S, plan.room()))) return rc;
     return run_q40_at(ctx, p, 3, plan, S, x_dev, (const uint8_t *)xq_dev);
 }
 
@@ -1438,7 +1441,7 @@ int spt_mul_q40_batch_into_host(spt_ctx *ctx, const spt_tensor *w, const float *
     p.resid = nullptr;
     const Q40Plan plan = q40_plan(&p, 1, in / 32, batch, false, xb + yb);
     char *S, *P;
-    if ((rc = arena(ctx, plan.total, &S)) || (rc = staging(ctx, xb + yb, &P))) return rc;
+    if ((rc = arena(ctx, plan.total, &S, plan.room())) || (rc = staging(ctx, xb + yb, &P))) return rc;
     p.y = (float *)(S + xb);
     memcpy(P, x_host, (size_t)x_len * 4);
     SPT_HIP(hipMemcpyAsync(S, P, (size_t)x_len * 4, hipMemcpyHostToDevice, ctx->stream));
