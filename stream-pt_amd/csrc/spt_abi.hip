@@ -162,8 +162,8 @@ hipError_t timed(spt_ctx *ctx, int kind, F &&launch) {
 }
 
 // Grow-only device scratch arena; returns a pointer to at least `bytes` bytes.
-// `more`: what the layer's next call is likely to ask for on top.
-int arena(spt_ctx *ctx, size_t bytes, char **out, size_t more = 0) {
+// `next`: what the layer's next call asks for, where that is known.
+int arena(spt_ctx *ctx, size_t bytes, char **out, size_t next = 0) {
     if (bytes > ctx->scratch_bytes) {
         if (ctx->scratch) {
             hipError_t e = hipStreamSynchronize(ctx->stream);
@@ -172,7 +172,7 @@ int arena(spt_ctx *ctx, size_t bytes, char **out, size_t more = 0) {
             ctx->scratch = nullptr;
             ctx->scratch_bytes = 0;
         }
-        const size_t want = bytes + std::max(bytes / 4, more) + 4096;
+        const size_t want = std::max(bytes + bytes / 4, next) + 4096;
         if (hipMalloc(&ctx->scratch, want) != hipSuccess) {
             ctx->scratch = nullptr;
             return fail(SPT_ERR_NOMEM, "cannot allocate %zu bytes of device scratch", want);
@@ -918,12 +918,6 @@ struct Q40Plan {
     bool views, dec, tile, gemm;
     int64_t nb, batch;
     size_t o_c, o_s, o_q, o_part, o_q34, total;
-    // A GEMM batch leaves room for its size again, up to 16 MB: O follows Q/K/V
-    // with an input that is often wider, and growing the arena waits for the
-    // stream and costs about 0.5 ms (740 us instead of 160 for such a layer's
-    // first pass). Smaller batches gain nothing: there the larger allocation
-    // alone was 45 us of a first pass of 90.
-    size_t room() const { return gemm ? std::min(total, size_t(16) << 20) : 0; }
 };
 
 Q40Plan q40_plan(const Q40Proj *p, int np, int64_t nb, int64_t batch, bool q8_in, size_t base) {
@@ -954,6 +948,24 @@ Q40Plan q40_plan(const Q40Proj *p, int np, int64_t nb, int64_t batch, bool q8_in
     L.o_q34 = c.take(L.tile && !q8_in ? batch * nb * spt::kQ80Block : 0);
     L.total = c.off;
     return L;
+}
+
+// What the output projection after Q/K/V takes of the arena (Q's rows wide, the
+// input's width of rows): Q/K/V's call leaves that much, for growing the arena
+// later waits for the stream and costs about 0.6 ms.  At 2880 -> 4096 / 512 /
+// 512 -> 2880 the quarter of slack holds it except at 193 to 320 tokens, where
+// only O splits K beside its views, and from 1,985, where nothing of Q/K/V
+// does.  First pass of a new context, norm to O, us, the call's own size again
+// (16 MB at most) as slack / this: 256 tokens 713 / 130, 320: 704 / 138, 1,999:
+// 325 / 325 (405 where O grew the arena); 65 to 192 and 321 to 1,984 within the
+// runs' spread (65: 85 / 87, 512: 141 / 140), with 0.62 to 0.88 of the memory.
+size_t q40_out_bytes(int64_t q_rows, int64_t in, int64_t batch) {
+    if (q_rows % 32 != 0) return 0;
+    const spt_tensor w{};
+    Q40Proj o{};
+    o.w = &w;
+    o.out = in;
+    return q40_plan(&o, 1, q_rows / 32, batch, false, 0).total;
 }
 
 // Quantize (x) or unpack (xq34) the input into the plan's views when it has
@@ -1360,7 +1372,7 @@ int spt_mul_q40_batch_bias_into(spt_ctx *ctx, const spt_tensor *w, const spt_ten
     p.resid = resid_dev;
     const Q40Plan plan = q40_plan(&p, 1, in / 32, batch, false, 0);
     char *S;
-    if ((rc = arena(ctx, plan.total, &S, plan.room()))) return rc;
+    if ((rc = arena(ctx, plan.total, &S))) return rc;
     return run_q40_at(ctx, &p, 1, plan, S, x_dev, nullptr);
 }
 
@@ -1379,7 +1391,7 @@ int spt_mul_q40_batch_q8_into(spt_ctx *ctx, const spt_tensor *w, const spt_tenso
     p.resid = resid_dev;
     const Q40Plan plan = q40_plan(&p, 1, in / 32, batch, true, 0);
     char *S;
-    if ((rc = arena(ctx, plan.total, &S, plan.room()))) return rc;
+    if ((rc = arena(ctx, plan.total, &S))) return rc;
     return run_q40_at(ctx, &p, 1, plan, S, nullptr, (const uint8_t *)xq_dev);
 }
 
@@ -1420,7 +1432,7 @@ int spt_mul_q40_qkv_batch_into(spt_ctx *ctx, const spt_tensor *w, const spt_tens
     if ((rc = check_device(ctx))) return rc;
     const Q40Plan plan = q40_plan(p, 3, in / 32, batch, xq_dev != nullptr, 0);
     char *S;
-    if ((rc = arena(ctx, plan.total, &S, plan.room()))) return rc;
+    if ((rc = arena(ctx, plan.total, &S, q40_out_bytes(p[0].out, in, batch)))) return rc;
     return run_q40_at(ctx, p, 3, plan, S, x_dev, (const uint8_t *)xq_dev);
 }
 
@@ -1441,7 +1453,7 @@ int spt_mul_q40_batch_into_host(spt_ctx *ctx, const spt_tensor *w, const float *
     p.resid = nullptr;
     const Q40Plan plan = q40_plan(&p, 1, in / 32, batch, false, xb + yb);
     char *S, *P;
-    if ((rc = arena(ctx, plan.total, &S, plan.room())) || (rc = staging(ctx, xb + yb, &P))) return rc;
+    if ((rc = arena(ctx, plan.total, &S)) || (rc = staging(ctx, xb + yb, &P))) return rc;
     p.y = (float *)(S + xb);
     memcpy(P, x_host, (size_t)x_len * 4);
     SPT_HIP(hipMemcpyAsync(S, P, (size_t)x_len * 4, hipMemcpyHostToDevice, ctx->stream));

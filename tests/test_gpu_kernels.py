@@ -388,10 +388,9 @@ def test_q40_split_batch_dependence(gpu_ctx, O):
 
 
 def spt_split(rows, ntok):
-    """The library's split rule (kQ40SplitMaxTiles = 256 tiles of 64 x 64,
-    narrow projections below 1024 rows always)."""
+    """The library's split rule (kQ40SplitMaxTiles = 256 tiles of 64 x 64)."""
     tiles = ((rows + 63) // 64) * ((ntok + 63) // 64)
-    return ntok >= 32 and (rows < 1024 or tiles < 256)
+    return ntok >= 32 and tiles < 256
 
 
 def _at_offset(raw, off):
@@ -504,3 +503,43 @@ def test_q40_views_of_fp32_and_blocks(gpu_ctx, O, batch):
     rows = [r for r in range(batch) if r not in (4, 5)]
     want = O.mul_q40_q8(w, np.ascontiguousarray(x[rows]).reshape(-1), din, dout, len(rows))
     assert_close(ah[rows].reshape(-1), want, what="Q4_0 from fp32")
+
+
+@pytest.mark.parametrize("batch", [29, 64, 65, 192, 193, 256, 320, 321, 512, 1985])
+def test_q40_arena_of_a_layer(batch):
+    """The arena that Q/K/V of a GPT-OSS layer make on a new context holds the
+    output projection that follows (it does not grow again), and is no larger
+    than the wider of the two calls needs: a quarter of slack on the views (40
+    bytes a block; 34 from the quantizer of the tiled form) and the split
+    projections' partial sums (16 bytes an output)."""
+    import torch
+
+    import spt
+    from spt import synth
+
+    H, Q, KV = 2880, 4096, 512
+
+    def need(nb, outs):
+        part = sum(16 * batch * o for o in outs if spt_split(o, batch))
+        return batch * nb * 40 + part + 1024
+
+    def weights(rows, cols):
+        w = torch.from_numpy(synth.q40_bytes(synth.stream_key(8, rows), rows, cols)).cuda()
+        return w, spt.Tensor.make("w", spt.TYPE_Q4_0, [cols, rows], w.data_ptr(), w.numel())
+
+    keep, ws = zip(*[weights(r, H) for r in (Q, KV, KV)])
+    wo, o = weights(H, Q)
+    x = torch.randn(batch * H, device="cuda")
+    c = torch.randn(batch * Q, device="cuda")
+    ys = [torch.empty(batch * r, device="cuda") for r in (Q, KV, KV)]
+    y = torch.empty(batch * H, device="cuda")
+    ctx = spt.Context(0, torch.cuda.current_stream().cuda_stream)
+    try:
+        ctx.mul_q40_qkv_batch_into(ws, None, x, ys, batch)
+        held = ctx.memory()[0]
+        ctx.mul_q40_batch_into(o, c, y, batch)
+        assert ctx.memory()[0] == held
+        assert held <= max(need(H // 32, (Q, KV, KV)) * 5 // 4, need(Q // 32, (H,))) + 4096
+        torch.cuda.synchronize()
+    finally:
+        ctx.close()
