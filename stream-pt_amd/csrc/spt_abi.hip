@@ -506,8 +506,9 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     if (use_gemm) {
         so.gm_start = (int32_t *)(S + L.o_gms);
         so.gm_grid = spt::mx_wide_grid();
-        so.wide_units[0] = (int32_t)(d / spt::kWideRows);
-        so.wide_units[1] = (int32_t)(h / spt::kWideRows);
+        const int64_t gate_up = spt::mx_wide_unit_rows((int)nbh), down = spt::mx_wide_unit_rows((int)nbd);
+        so.wide_units[0] = (int32_t)((d + gate_up - 1) / gate_up);
+        so.wide_units[1] = (int32_t)((h + down - 1) / down);
     }
     // the two grouped GEMV launches' start table, for their grids
     const int slots = (int)(n < E ? n : E);
@@ -957,7 +958,7 @@ Q40Plan q40_plan(const Q40Proj *p, int np, int64_t nb, int64_t batch, bool q8_in
 // only O splits K beside its views, and from 1,985, where nothing of Q/K/V
 // does.  First pass of a new context, norm to O, us, the call's own size again
 // (16 MB at most) as slack / this: 256 tokens 713 / 130, 320: 704 / 138, 1,999:
-// 325 / 325 (405 where O grew the arena); 65 to 192 and 321 to 1,984 within the
+// 325 / 325; 65 to 192 and 321 to 1,984 within the
 // runs' spread (65: 85 / 87, 512: 141 / 140), with 0.62 to 0.88 of the memory.
 size_t q40_out_bytes(int64_t q_rows, int64_t in, int64_t batch) {
     if (q_rows % 32 != 0) return 0;

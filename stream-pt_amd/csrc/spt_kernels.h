@@ -283,8 +283,10 @@ int device_cus();
 hipError_t launch_mx_mfma(hipStream_t s, GemvMode mode, const MxMfmaArgs &a, int slots);
 // The grid launch_mx_mfma uses for these arguments (0: nothing to launch).
 int mx_mfma_grid(GemvMode mode, const MxMfmaArgs &a, int slots);
-// The grid of launch_mx_wide (SelectOut::gm_grid).
+// The grid of launch_mx_wide (SelectOut::gm_grid), and the output rows of its
+// units for an input of nb blocks (SelectOut::wide_units).
 int mx_wide_grid();
+int mx_wide_unit_rows(int nb);
 // Whether the wide launches take expert matrices of this many bytes (their
 // loads use offsets past 2^31 for "nothing").
 inline bool mx_wide_fits(uint64_t expert_bytes) { return expert_bytes <= 0x7FFFFF00ull; }

@@ -53,8 +53,8 @@ constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kStages = 3;
 constexpr int kMaxPart = 45;         // blocks of a row per stage
+constexpr int kMaxQuarter = 20;      // the same with two row tiles a step
 constexpr int kLoadWaves = 4;        // waves that issue the loads (one per SIMD)
-constexpr int kLoadsMax = 7;         // 1 KB DMA loads per such wave and stage
 constexpr int kPartsLds = kWaves * kWideRows * kGemmTokens * 4;  // the waves' partial sums of a step
 constexpr int kStaticLds = 20 * 1024;  // static LDS of a workgroup, at most
 constexpr int kDownStores = 1, kActStores = 4;  // vector stores of an epilogue that stores (down; up step)
@@ -62,35 +62,43 @@ constexpr int kBiasWave = kLoadWaves - 1;  // loads the biases
 constexpr int kEMin = 4, kEMax = 240;
 constexpr int kXcds = 8;
 constexpr uint32_t kOOR = 0x80000000u;  // buffer offset past every range: reads zero
+constexpr int kVmcnt0 = 0x0F70;          // s_waitcnt vmcnt(0)
 // 16-byte slots of a row's window in a stage: its blocks and up to 15 bytes
 // before them; an odd number, so that 16 rows begin at 16 different groups of
 // banks (2,560 inputs, 40 blocks a part: down of 105 experts 251 us with 44
 // slots a row, every fourth row in the same banks).
 __host__ __device__ constexpr int row_slots(int blocks) { return ((blocks * kMxBlock + 15 + 15) / 16) | 1; }
-__host__ __device__ constexpr int stage_loads(int blocks) { return (kWideRows * row_slots(blocks) + 63) / 64; }
-// Row slot p of a stage holds row slot_row(p), row r lies in row_slot(r): rows
-// 16-31 are rotated by one, so that the two rows whose slots are 16 apart (the
-// same LDS banks) begin at different bytes of their first 16 (with 2,880
-// inputs a row is 10 bytes past a multiple of 16) and the 32 lanes' reads
-// meet no bank twice.
-__device__ inline int slot_row(int p) { return p < 16 ? p : 16 + ((p + 1) & 15); }
+// 1 KB DMA loads of a stage of RT row tiles, and of each loading wave (the last
+// of those waves has one fewer: the bias in its place).
+template <int RT>
+__host__ __device__ constexpr int stage_loads(int blocks) { return (RT * kWideRows * row_slots(blocks) + 63) / 64; }
+template <int RT>
+__host__ __device__ constexpr int wave_loads(int blocks) { return (stage_loads<RT>(blocks) + 1 + kLoadWaves - 1) / kLoadWaves; }
+// Row slot p of a stage holds row slot_row(p), row r of a tile lies in its slot
+// row_slot(r): rows 16-31 of a tile are rotated by one, so that the two rows
+// whose slots are 16 apart (the same LDS banks) begin at different bytes of
+// their first 16 (with 2,880 inputs a row is 10 bytes past a multiple of 16) and
+// the 32 lanes' reads meet no bank twice.
+__device__ inline int slot_row(int p) { return (p & 16) == 0 ? p : (p & ~15) + ((p + 1) & 15); }
 __device__ inline int row_slot(int r) { return r < 16 ? r : 16 + ((r - 1) & 15); }
-static_assert(stage_loads(kMaxPart) <= kLoadWaves * kLoadsMax, "stage loads");
-static_assert(stage_loads(kMaxPart) <= kBiasWave + kLoadWaves * (kLoadsMax - 1), "the bias wave has one load fewer");
 static_assert(2 * kMaxPart >= kMxMaxInput / 32, "a row is at most two parts");
-static_assert(kStages * 1024 * stage_loads(kMaxPart) + kPartsLds + kStaticLds <= 160 * 1024, "LDS");
+// dynamic LDS of a workgroup: the stages and the waves' partial sums
+template <int RT>
+constexpr int dynamic_lds(int blocks) { return kStages * 1024 * stage_loads<RT>(blocks) + kPartsLds; }
+static_assert(dynamic_lds<1>(kMaxPart) + kStaticLds <= 160 * 1024, "LDS");
+static_assert(dynamic_lds<2>(kMaxQuarter) + kStaticLds + 6 * 1024 <= 160 * 1024, "LDS with two row tiles");
 static_assert(kGemmTokens == 64, "two 32-entry tiles per pass");
 
 // Waits for a stage (the waves that load; the barrier after it does for the
-// others): at most the kLoadsMax loads of the stage issued after it
-// and the N stores of one epilogue may be outstanding.  The counter retires
+// others): at most N operations may be outstanding, the loads of the stage
+// issued after it and the stores of one epilogue.  The counter retires
 // in order, so every wave must issue exactly these since (anything more only
 // makes the wait longer): loads and stores are never skipped by a branch but
 // given an offset past the range.
 template <int N>
 __device__ __attribute__((always_inline)) inline void wait_stage(int wave) {
     if (wave < kLoadWaves)
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kLoadsMax + N) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
     else
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
@@ -184,35 +192,41 @@ __device__ float lut_dot(const ByteView &v, uint32_t row_pos, int nb, const int8
 
 }  // namespace
 
-// Persistent workgroups of eight waves, one per CU.  A unit is 32 outputs:
-// gate/up takes it in two steps (its 32 gate rows, then its 32 up rows),
+// Persistent workgroups of eight waves, one per CU.  A unit is RT tiles of 32
+// outputs: gate/up takes it in two steps (its gate rows, then its up rows),
 // down in one.  The packing deals each workgroup a contiguous range of
 // (expert, pass of 64 entries, unit) whose cost is its share of the whole
 // (k_pack), so a workgroup changes pass once or twice in a launch.
 //
-// The eight waves split K, not the rows or the entries: within each part of
-// a row wave w multiplies blocks w, w + 8, ..., so its B digits for all 64
-// entries stay in registers for the whole pass (P * NJ blocks x 2 tiles x 6
-// VGPRs) and every weight byte is read from LDS once.  Weights come by LDS
-// DMA in stages of one part (half a row beyond 45 blocks) of 32 rows -- a
-// ring of three stages, two in flight while one is multiplied; a row's part
-// is contiguous in memory, so a stage is 32 runs of up to 765 bytes.
+// The eight waves split K, not the entries: within each part of a row wave w
+// multiplies blocks w, w + 8, ..., so its B digits for all 64 entries stay in
+// registers for the whole pass (P * NJ blocks x 2 tiles x 6 VGPRs) and every
+// weight byte is read from LDS once.  Short rows leave a wave a block or two of
+// that: with RT = 2 four waves split K on the first 32 rows of a step, four on
+// the next (the last step's second tile may lie past the rows: its results go
+// nowhere).  Weights come by LDS DMA in stages of one part (half a row beyond
+// 45 blocks) of a step's rows -- a ring of three stages, two in flight while one
+// is multiplied; a row's part is contiguous in memory, so a stage is 32 or 64
+// runs of up to 765 bytes.
 //
-// The waves' partial sums of a step meet in LDS, and each output's eight
-// partials are added in wave order, so it does not depend on its entry's
-// place in the list.  A wave takes eight entries of a two-tile pass (four of
-// a one-tile pass), all 32 rows, so a 32-element Q8_0 block of act stays
+// The waves' partial sums of a step meet in LDS, and each output's partials
+// (eight, or four with RT = 2) are added in wave order, so it does not depend
+// on its entry's place in the list.  A wave takes eight entries of a two-tile pass (four of
+// a one-tile pass), all 32 rows of a tile, so a 32-element Q8_0 block of act stays
 // within it.  This epilogue of a step runs at the start of the next one.
-template <int MODE, int P, int NJ>
+template <int MODE, int P, int NJ, int RT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_mx_wide(MxWideArgs) {
+    constexpr int kSub = MODE == kGateUp ? 2 : 1;  // steps per unit
+    constexpr int KS = kWaves / RT, kStepRows = RT * kWideRows;  // parts of K; rows of a step
+    constexpr int kLoads = wave_loads<RT>(NJ * KS < kMaxPart ? NJ * KS : kMaxPart);
+    static_assert(RT == 1 || P == 1, "rows in parts: one row tile");
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ uint32_t s_bias[8][64];      // raw bias dwords of a step's rows
     __shared__ int s_ent[2][kGemmTokens];   // per pass parity: list entries (-1 past the end)
-    __shared__ uint32_t s_apos[kLoadsMax][64 * kLoadWaves];  // each loading thread's offsets of a stage
-    __shared__ v4f s_gate[MODE == kGateUp ? kThreads : 1];  // gate sums of a unit, for its up step
+    __shared__ uint32_t s_apos[kLoads][64 * kLoadWaves];  // each loading thread's offsets of a stage
+    __shared__ v4f s_gate[MODE == kGateUp ? RT * kThreads : 1];  // gate sums of a unit, for its up step
     __shared__ uint32_t s_spare[256];       // where the loads past a stage's go
-    __shared__ uint32_t s_special[2];       // per step parity: rows with special scales
-    constexpr int kSub = MODE == kGateUp ? 2 : 1;  // steps per unit
+    __shared__ uint32_t s_special[2][RT];   // per step parity and row tile: rows with special scales
 
     WideArgs *const args = (WideArgs *)__builtin_amdgcn_kernarg_segment_ptr();
     WideArgs &a = wide_args(args);
@@ -226,7 +240,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         asm volatile("" : "+v"(l));
         return l;
     };
-    const int nb = a.nb, units = a.rows / kWideRows;
+    const int kp = RT == 1 ? wave : wave % KS, rt = RT == 1 ? 0 : wave / KS;  // the wave's part of K and row tile
+    const int nb = a.nb, units = (a.rows + kStepRows - 1) / kStepRows;
     const uint32_t row_bytes = (uint32_t)nb * kMxBlock;
     const int G = gridDim.x;
     // the ranges are dealt XCD-major (workgroup b runs on XCD b % 8), so
@@ -248,13 +263,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     // piece q % slots)
     const int nb0 = P == 1 ? nb : (nb + 1) / 2;
     const int slots = row_slots(nb0);
-    const int nloads = stage_loads(nb0);
+    const int nloads = stage_loads<RT>(nb0);
     const uint32_t stage_bytes = 1024u * (uint32_t)nloads;
 #pragma unroll
-    for (int k = 0; k < kLoadsMax; k++) {
+    for (int k = 0; k < kLoads; k++) {
         if (wave >= kLoadWaves) break;
         const int q = 64 * (wave + kLoadWaves * k) + lane, r = q / slots, pc = q - r * slots;
-        s_apos[k][tid] = r < kWideRows ? (uint32_t)slot_row(r) * row_bytes + 16u * (uint32_t)pc : kOOR;
+        s_apos[k][tid] = r < kStepRows ? (uint32_t)slot_row(r) * row_bytes + 16u * (uint32_t)pc : kOOR;
     }
     typedef __attribute__((address_space(3))) uint8_t lds_u8;
     typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
@@ -262,7 +277,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const uint32_t bias0 = (uint32_t)reinterpret_cast<uintptr_t>((lds_u8 *)&s_bias[0][0]);
     const uint32_t spare0 = (uint32_t)reinterpret_cast<uintptr_t>((lds_u8 *)&s_spare[0]);
     uint8_t *parts = lds + kStages * stage_bytes;
-    if (tid < 2) s_special[tid] = 0u;
+    if (tid < 2 * RT) (&s_special[0][0])[tid] = 0u;
 
     // ---- the issue side: walks ahead of the multiply -----------------------
     Walk iw = cur;
@@ -296,9 +311,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const uintptr_t bb = reinterpret_cast<uintptr_t>(a.bias[m]);
         const uint32_t lead = (uint32_t)(bb & 3u);
         const u32x4v rb = rsrc_words(reinterpret_cast<const void *>(bb - lead), a.bias[m] ? (uint32_t)((a.bias_bytes[m] + lead + 3u) & ~3ull) : 0u);
-        const uint32_t idx = (uint32_t)iw.e * (uint32_t)a.rows + (uint32_t)(iw.u * kWideRows + (ln & 31));
+        const uint32_t idx = (uint32_t)iw.e * (uint32_t)a.rows + (uint32_t)(iw.u * kStepRows + (ln & (kStepRows - 1)));
         const uint32_t off = (lead + idx * (a.bias_type[m] == 0 ? 4u : 2u)) & ~3u;
-        dma4(rb, bias0 + 256u * (uint32_t)(i_step & 7), i_left > 0 && ln < 32 ? off : kOOR, 0u);
+        dma4(rb, bias0 + 256u * (uint32_t)(i_step & 7), i_left > 0 && ln < kStepRows ? off : kOOR, 0u);
     };
     // after them: on to the next stage
     auto issue_end = [&]() SPT_INLINE {
@@ -331,15 +346,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         // from the 16-byte boundary at or below the matrix to the one at or
         // above its end
         const u32x4v rs = rsrc_words(reinterpret_cast<const void *>(mb - le), (expert_bytes + le + 15u) & ~15u);
-        const uint32_t adv = i_left > 0 ? le + (uint32_t)(iw.u * kWideRows) * row_bytes + (P == 2 && i_part ? (uint32_t)nb0 * kMxBlock : 0u) : kOOR;
+        const uint32_t adv = i_left > 0 ? le + (uint32_t)(iw.u * kStepRows) * row_bytes + (P == 2 && i_part ? (uint32_t)nb0 * kMxBlock : 0u) : kOOR;
         const int ln = lane_now();
 #pragma unroll
-        for (int k = 0; k < kLoadsMax - 1; k++) issue_load(rs, k, adv, ln);
+        for (int k = 0; k < kLoads - 1; k++) issue_load(rs, k, adv, ln);
         // the last loading wave has one load fewer (kBiasWave): the bias in its place
         if (wave == kBiasWave && i_part == 0)
             issue_bias(ln);
         else
-            issue_load(rs, kLoadsMax - 1, adv, ln);
+            issue_load(rs, kLoads - 1, adv, ln);
         issue_end();
     };
     issue();
@@ -364,24 +379,39 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             const int ent = a.list[base + (32 * t + l32 < nt ? 32 * t + l32 : 0)];
             tpos[t] = (uint32_t)(MODE == kGateUp ? ent / a.topk : ent) * (uint32_t)nb * (uint32_t)kDigitBytes;
         }
+        // A block's two 16-byte pieces lie in one 64-byte line: they are asked
+        // for together (every block's first piece before any second one fetched
+        // the lines twice: down at 2,000 tokens 264.7 -> 267.1 us).
+        uint32_t d[P][NJ][2];
 #pragma unroll
         for (int p = 0; p < P; p++)
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
-                const int bl = wave + kWaves * j;
-                const bool ok = bl < (p ? nb - nb0 : nb0);
-                float d[2];
+                const int so = KS * kDigitBytes * j;
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
                     // (past the part: some block's digits, or zeros, with d_x = 0)
-                    const uint32_t o = tpos[t] + (uint32_t)((p * nb0 + wave) * kDigitBytes);
-                    const int so = kWaves * kDigitBytes * j;
+                    const uint32_t o = tpos[t] + (uint32_t)((p * nb0 + kp) * kDigitBytes);
                     const u32x4 lo = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rt, o + 16u * (uint32_t)half + so, 0, 0));
                     const u32x4 hi = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rt, o + 16u * (uint32_t)half + 32u + so, 0, 0));
                     B[p][j][t] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, 0, 0};
-                    d[t] = ok ? __uint_as_float(hi.z) : 0.0f;
+                    d[p][j][t] = hi.z;
                 }
-                dx[p][j] = f16x2{(_Float16)d[0], (_Float16)d[1]};  // exact: d_x is an fp16 value
+                asm volatile("" ::: "memory");
+            }
+        // All of it arrives here: waited for where the products use it, the
+        // compiler's waits of every later step would drain the loads of the next
+        // stages too (512 tokens, Zipf(1.1): gate/up 179.9 -> 178.1 us).
+        __builtin_amdgcn_s_waitcnt(kVmcnt0);
+#pragma unroll
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const bool ok = kp + KS * j < (p ? nb - nb0 : nb0);
+                asm volatile("" : "+v"(d[p][j][0]), "+v"(d[p][j][1])::"memory");
+                // exact: d_x is an fp16 value
+                dx[p][j] = f16x2{(_Float16)(ok ? __uint_as_float(d[p][j][0]) : 0.0f), (_Float16)(ok ? __uint_as_float(d[p][j][1]) : 0.0f)};
+                asm volatile("" : "+v"(dx[p][j]));
             }
     };
 
@@ -392,8 +422,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         constexpr int NT = decltype(nt_c)::value, p = decltype(p_c)::value;
         const int ln = lane_now(), l32 = ln & 31;
         const int sb = ln < 32 ? 134 : 130;  // B scale: digit / 8, times 16 for h
-        const uint32_t pos = lds0 + (uint32_t)stage * stage_bytes + (uint32_t)(row_slot(l32) * slots) * 16u + lead +
-                             (uint32_t)(wave * kMxBlock);
+        const uint32_t pos = lds0 + (uint32_t)stage * stage_bytes + (uint32_t)((kWideRows * rt + row_slot(l32)) * slots) * 16u + lead +
+                             (uint32_t)(kp * kMxBlock);
         lds_cu32 *pa = reinterpret_cast<lds_cu32 *>((uintptr_t)(pos & ~3u));
         const uint32_t sel = 0x04030201u + (pos & 3u) * 0x01010101u, esh = (pos & 3u) * 8u;
         const int cnt = p ? nb - nb0 : nb0;
@@ -402,18 +432,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int i = 0; i < 5; i++) d[i] = pa[i];
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const bool ok = wave + kWaves * j < cnt;
+            const bool ok = kp + KS * j < cnt;
             const uint32_t e = __builtin_amdgcn_ubfe(d[0], esh, 8u);
             emin = min(emin, ok ? e : 127u);
             emax = max(emax, ok ? e : 127u);
             const int sa = ok ? (int)e : 127;  // past the part: d_x = 0 times a finite value
             const v8i A = {(int)__builtin_amdgcn_perm(d[1], d[0], sel), (int)__builtin_amdgcn_perm(d[2], d[1], sel),
                            (int)__builtin_amdgcn_perm(d[3], d[2], sel), (int)__builtin_amdgcn_perm(d[4], d[3], sel), 0, 0, 0, 0};
-            // the next block's reads fly during this one's products; blocks 8
-            // apart are 136 bytes (34 dwords) apart: one alignment
+            // the next block's reads fly during this one's products; blocks KS
+            // (4 or 8) apart are 17 or 34 dwords apart: one alignment
             if (j + 1 < NJ) {
 #pragma unroll
-                for (int i = 0; i < 5; i++) d[i] = pa[34 * (j + 1) + i];
+                for (int i = 0; i < 5; i++) d[i] = pa[KS * kMxBlock / 4 * (j + 1) + i];
             }
             const v16f z = {};
 #pragma unroll
@@ -429,34 +459,36 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
     // ---- the epilogue of the previous step ---------------------------------------
     int q_u = 0, q_e = 0, q_sub = 0, q_par = 0, q_ntile = 0, q_step = 0;
-    // NT tiles: lane l of wave v takes TW = 4 NT entries' rows, R = 2 NT rows
-    // each: entry TW * v + l % TW, rows R * (l / TW) .. + R - 1.
-    auto epilogue_of = [&](auto nt_c) SPT_INLINE {
-        constexpr int NT = decltype(nt_c)::value, TW = 4 * NT, R = 2 * NT;
+    // NT tiles, row tile S: lane l of wave v takes TW = 4 NT entries' rows, R =
+    // 2 NT rows each: entry TW * v + l % TW, rows R * (l / TW) .. + R - 1.
+    auto epilogue_of = [&](auto nt_c, auto s_c) SPT_INLINE {
+        constexpr int NT = decltype(nt_c)::value, S = decltype(s_c)::value, TW = 4 * NT, R = 2 * NT;
         typedef float vRf __attribute__((ext_vector_type(R)));
         typedef uint32_t vRu __attribute__((ext_vector_type(R)));
         WideArgs &a = wide_args(args);
         const int ln = lane_now(), t = TW * wave + (ln & (TW - 1)), r0 = R * (ln / TW);
-        const vRf *pp = reinterpret_cast<const vRf *>(parts + part_slot(t >> 5, r0 >> 2, t & 31) * 16 + 4 * (r0 & 3));
-        vRf y[kWaves];
+        const int tile = q_u * RT + S;  // of 32 rows
+        const vRf *pp = reinterpret_cast<const vRf *>(parts + S * KS * (kPartsLds / kWaves) + part_slot(t >> 5, r0 >> 2, t & 31) * 16 + 4 * (r0 & 3));
+        vRf y[KS];
 #pragma unroll
-        for (int w = 0; w < kWaves; w++) y[w] = pp[w * (kPartsLds / kWaves / (4 * R))];
+        for (int w = 0; w < KS; w++) y[w] = pp[w * (kPartsLds / kWaves / (4 * R))];
         const int m = MODE == kGateUp ? q_sub : 0;
-        const vRu braw = *reinterpret_cast<const vRu *>(&s_bias[q_step & 7][r0]);
+        const vRu braw = *reinterpret_cast<const vRu *>(&s_bias[q_step & 7][kWideRows * S + r0]);
         vRf s = y[0];
 #pragma unroll
-        for (int w = 1; w < kWaves; w++)
+        for (int w = 1; w < KS; w++)
 #pragma unroll
             for (int i = 0; i < R; i++) s[i] += y[w][i];
-        const int ent = s_ent[q_par][t];
-        const uint32_t spec = s_special[q_step & 1];
+        // (a last step's tile past the rows goes nowhere)
+        const int ent = RT == 1 || tile * kWideRows < a.rows ? s_ent[q_par][t] : -1;
+        const uint32_t spec = s_special[q_step & 1][S];
         if (spec && ent >= 0) {
             const ByteView cv = make_view((MODE == kGateUp && q_sub ? a.w[1] : a.w[0]) + (uint64_t)q_e * a.expert_bytes,
                                           a.expert_bytes);
             const size_t ar = MODE == kGateUp ? ent / a.topk : ent;
             for (int i = 0; i < R; i++) {
                 if (!((spec >> (r0 + i)) & 1u)) continue;
-                const float v = lut_dot(cv, (uint32_t)(q_u * kWideRows + r0 + i) * row_bytes, nb, a.codes + ar * nb * 32,
+                const float v = lut_dot(cv, (uint32_t)(tile * kWideRows + r0 + i) * row_bytes, nb, a.codes + ar * nb * 32,
                                         a.tab + ar * nb * kDigitBytes);
 #pragma unroll
                 for (int k = 0; k < R; k++) s[k] = k == i ? v : s[k];
@@ -478,7 +510,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         }
         if constexpr (MODE == kDown) {
             const rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(a.out, (short)0, (int)kOOR, kRsrcWord3);
-            const uint32_t o = ent < 0 ? kOOR : ((uint32_t)ent * (uint32_t)a.rows + (uint32_t)(q_u * kWideRows + r0)) * 4u;
+            const uint32_t o = ent < 0 ? kOOR : ((uint32_t)ent * (uint32_t)a.rows + (uint32_t)(tile * kWideRows + r0)) * 4u;
             if constexpr (R == 4)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4s, s), ro, o, 0, 0);
             else
@@ -486,7 +518,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             return;
         }
         // (a gate sum is read back by the thread that wrote it, in the same pass)
-        vRf &gate = *reinterpret_cast<vRf *>(&s_gate[64 * wave + ln]);
+        vRf &gate = *reinterpret_cast<vRf *>(&s_gate[kThreads * S + 64 * wave + ln]);
         if (q_sub == 0) {
             gate = s;
             return;
@@ -535,7 +567,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         // Four stores, always: codes, the two pieces of the digits (which begin
         // at 3 R/2 bytes times an odd or even number: the 16-bit or 8-bit piece
         // first where odd) and the scale.
-        const uint32_t blk = (uint32_t)ent * (uint32_t)(a.rows / kWideRows) + (uint32_t)q_u;
+        const uint32_t blk = (uint32_t)ent * (uint32_t)(a.rows / kWideRows) + (uint32_t)tile;
         const rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(a.act_codes, (short)0, (int)kOOR, kRsrcWord3);
         const rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(a.act_tab, (short)0, (int)kOOR, kRsrcWord3);
         const uint32_t oc = ent < 0 ? kOOR : blk * 32u + (uint32_t)r0, ot = ent < 0 ? kOOR : blk * (uint32_t)kDigitBytes;
@@ -552,7 +584,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         }
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(f16_bits_to_f32(dh)), rt, (r0 & 15) == 0 ? ot + digit_scale(g) : kOOR, 0, 0);
         if (ent >= 0 && (a.tap[0] || a.tap[1] || a.out || a.act_blocks34)) {
-            const size_t o = (size_t)ent * a.rows + q_u * kWideRows + r0;
+            const size_t o = (size_t)ent * a.rows + tile * kWideRows + r0;
             if (a.tap[0]) *reinterpret_cast<vRf *>(a.tap[0] + o) = gv;
             if (a.tap[1]) *reinterpret_cast<vRf *>(a.tap[1] + o) = s;
             if (a.out) *reinterpret_cast<vRf *>(a.out + o) = act;
@@ -567,11 +599,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             }
         }
     };
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    using C2 = std::integral_constant<int, 2>;
     auto epilogue = [&]() SPT_INLINE {
-        if (q_ntile == 2)
-            epilogue_of(std::integral_constant<int, 2>{});
-        else
-            epilogue_of(std::integral_constant<int, 1>{});
+        if (q_ntile == 2) {
+            epilogue_of(C2{}, C0{});
+            if constexpr (RT == 2) epilogue_of(C2{}, C1{});
+        } else {
+            epilogue_of(C1{}, C0{});
+            if constexpr (RT == 2) epilogue_of(C1{}, C1{});
+        }
     };
 
     // ---- the steps -----------------------------------------------------------------
@@ -582,11 +620,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         // since this stage's loads: the next stage's, and the epilogue of step - 2
         // (which stored if it was an up step, as this one then is)
         if (MODE == kDown && step > 1)
-            wait_stage<kDownStores>(wave);
+            wait_stage<kLoads + RT * kDownStores>(wave);
         else if (MODE == kGateUp && step > 1 && sub == 1)
-            wait_stage<kActStores>(wave);
+            wait_stage<kLoads + RT * kActStores>(wave);
         else
-            wait_stage<0>(wave);
+            wait_stage<kLoads>(wave);
         raw_barrier();  // this stage has landed; the previous step's partial sums are in place
         issue();
         if (step > 0) epilogue();
@@ -594,16 +632,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             load_pass();
             fresh = false;
         }
-        const uint32_t rpos = (kSub == 2 && sub ? c_le[kSub - 1] : c_le[0]) + (uint32_t)(cur.u * kWideRows + (lane_now() & 31)) * row_bytes;
+        const uint32_t rpos = (kSub == 2 && sub ? c_le[kSub - 1] : c_le[0]) + (uint32_t)(cur.u * kStepRows + kWideRows * rt + (lane_now() & 31)) * row_bytes;
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
         emin = 127u;
         emax = 127u;
-        using C0 = std::integral_constant<int, 0>;
-        using C1 = std::integral_constant<int, 1>;
-        using C2 = std::integral_constant<int, 2>;
         if (ntile == 2)
             multiply(C2{}, C0{}, stage, rpos & 15u);
         else
@@ -612,14 +647,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         if constexpr (P == 2) {
             // since: the next stage's loads and the epilogue of step - 1
             if (MODE == kDown && step > 0)
-                wait_stage<kDownStores>(wave);
+                wait_stage<kLoads + RT * kDownStores>(wave);
             else if (MODE == kGateUp && step > 0 && sub == 0)
-                wait_stage<kActStores>(wave);
+                wait_stage<kLoads + RT * kActStores>(wave);
             else
-                wait_stage<0>(wave);
+                wait_stage<kLoads>(wave);
             raw_barrier();  // this stage; every wave is past the epilogue
             issue();
-            if (step > 0 && tid == 0) s_special[q_step & 1] = 0u;
+            if (step > 0 && tid < RT) s_special[q_step & 1][tid] = 0u;
             const uint32_t lead = (rpos + (uint32_t)nb0 * kMxBlock) & 15u;
             if (ntile == 2)
                 multiply(C2{}, C1{}, stage, lead);
@@ -629,7 +664,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         } else {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             raw_barrier();  // every wave is past the epilogue
-            if (step > 0 && tid == 0) s_special[q_step & 1] = 0u;
+            if (step > 0 && tid < RT) s_special[q_step & 1][tid] = 0u;
         }
         const int ln = lane_now();
 #pragma unroll
@@ -642,7 +677,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             }
         }
         const uint64_t sm = __ballot(emin < (uint32_t)kEMin || emax > (uint32_t)kEMax);
-        if (sm && ln == 0) atomicOr(&s_special[step & 1], (uint32_t)sm | (uint32_t)(sm >> 32));
+        if (sm && ln == 0) atomicOr(&s_special[step & 1][rt], (uint32_t)sm | (uint32_t)(sm >> 32));
         q_u = cur.u;
         q_e = cur.e;
         q_sub = sub;
@@ -671,42 +706,54 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
 int mx_wide_grid() { return device_cus(); }
 
+template <int MODE, int P, int NJ, int RT>
+static hipError_t launch_wide_form(hipStream_t s, const MxWideArgs &a, int nb0) {
+    // one-time opt-in to more than 64 KB of dynamic LDS
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mx_wide<MODE, P, NJ, RT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       dynamic_lds<RT>(RT == 2 ? kMaxQuarter : kMaxPart));
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((k_mx_wide<MODE, P, NJ, RT>), dim3(mx_wide_grid()), dim3(kThreads), dynamic_lds<RT>(nb0), s, a);
+    return hipGetLastError();
+}
+
+// Rows of a step of a launch over rows of nb blocks: two row tiles as long as
+// their stages fit the LDS.  A step's exchange of partial sums, its barriers and
+// the start of its loads cost about 4,000 cycles however short the rows are (at
+// 90 blocks the whole step is 10,000).  Gate/up of 128 experts, 12 entries each,
+// us, one tile / two: 512 inputs x 2,880 rows 189 / 149; down 2,880 inputs' 512:
+// 64 / 50; 512 x 512, six entries: 33.0 / 28.1.
+int mx_wide_unit_rows(int nb) { return nb <= kMaxQuarter ? 2 * kWideRows : kWideRows; }
+
+// The form with exactly the blocks per wave and part of this row, rounded up:
+// a block past the part costs its products, a load past the stage's its issue
+// (1,536 inputs, 24 blocks a part, 128 experts: gate/up and down 162 + 77 us with
+// four blocks a wave and 28 loads a stage, 139 + 64 with three and 15).
 template <int MODE>
 static hipError_t launch_wide_mode(hipStream_t s, const MxWideArgs &a) {
-    const int nb0 = a.nb <= kMaxPart ? a.nb : (a.nb + 1) / 2;
-    const size_t lds = (size_t)kStages * 1024 * stage_loads(nb0) + kPartsLds;
-    constexpr int kLdsMax = kStages * 1024 * stage_loads(kMaxPart) + kPartsLds;
-    // one-time opt-in to more than 64 KB of dynamic LDS
-    static const hipError_t attr = [] {
-        const void *f[] = {reinterpret_cast<const void *>(&k_mx_wide<MODE, 1, 3>), reinterpret_cast<const void *>(&k_mx_wide<MODE, 1, 4>),
-                           reinterpret_cast<const void *>(&k_mx_wide<MODE, 1, 6>), reinterpret_cast<const void *>(&k_mx_wide<MODE, 2, 4>),
-                           reinterpret_cast<const void *>(&k_mx_wide<MODE, 2, 5>), reinterpret_cast<const void *>(&k_mx_wide<MODE, 2, 6>)};
-        hipError_t e = hipSuccess;
-        for (const void *k : f)
-            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
-        return e;
-    }();
-    if (attr != hipSuccess) return attr;
-    const dim3 grid(mx_wide_grid()), block(kThreads);
-    // blocks per wave and part, rounded up
-    const int nj = (nb0 + kWaves - 1) / kWaves;
-    auto launch = [&](auto *k) { hipLaunchKernelGGL(k, grid, block, lds, s, a); };
-    if (a.nb <= kMaxPart) {
-        if (nj <= 3)
-            launch(k_mx_wide<MODE, 1, 3>);
-        else if (nj <= 4)
-            launch(k_mx_wide<MODE, 1, 4>);
-        else
-            launch(k_mx_wide<MODE, 1, 6>);
-    } else {
-        if (nj <= 4)
-            launch(k_mx_wide<MODE, 2, 4>);
-        else if (nj <= 5)
-            launch(k_mx_wide<MODE, 2, 5>);
-        else
-            launch(k_mx_wide<MODE, 2, 6>);
+    if (a.nb <= kMaxQuarter) {
+        switch ((a.nb + 3) / 4) {
+        case 1:
+        case 2: return launch_wide_form<MODE, 1, 2, 2>(s, a, a.nb);
+        case 3: return launch_wide_form<MODE, 1, 3, 2>(s, a, a.nb);
+        case 4: return launch_wide_form<MODE, 1, 4, 2>(s, a, a.nb);
+        default: return launch_wide_form<MODE, 1, 5, 2>(s, a, a.nb);
+        }
     }
-    return hipGetLastError();
+    const int nb0 = a.nb <= kMaxPart ? a.nb : (a.nb + 1) / 2, nj = (nb0 + kWaves - 1) / kWaves;
+    if (a.nb <= kMaxPart) {
+        switch (nj) {
+        case 3: return launch_wide_form<MODE, 1, 3, 1>(s, a, nb0);
+        case 4: return launch_wide_form<MODE, 1, 4, 1>(s, a, nb0);
+        case 5: return launch_wide_form<MODE, 1, 5, 1>(s, a, nb0);
+        default: return launch_wide_form<MODE, 1, 6, 1>(s, a, nb0);
+        }
+    }
+    switch (nj) {
+    case 3: return launch_wide_form<MODE, 2, 3, 1>(s, a, nb0);
+    case 4: return launch_wide_form<MODE, 2, 4, 1>(s, a, nb0);
+    case 5: return launch_wide_form<MODE, 2, 5, 1>(s, a, nb0);
+    default: return launch_wide_form<MODE, 2, 6, 1>(s, a, nb0);
+    }
 }
 
 hipError_t launch_mx_wide(hipStream_t s, GemvMode mode, const MxWideArgs &a) {

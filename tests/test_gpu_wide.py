@@ -110,3 +110,15 @@ def test_route_wide_bits(gpu_ctx, O, hidden, experts, batch):
     want = O.route(w.reshape(-1), b, np.ascontiguousarray(x[rows]).reshape(-1), len(rows), hidden, experts)
     got = out.cpu().numpy().reshape(batch, experts)[rows]
     assert np.array_equal(bits(got.reshape(-1)), bits(np.asarray(want, np.float32).reshape(-1)))
+
+
+@pytest.mark.parametrize("hidden,dim", [(128, 160), (256, 288), (384, 416), (512, 544), (640, 672),
+                                        (768, 800), (1024, 1056), (1280, 1312),
+                                        (1472, 1536), (1568, 2048), (2080, 2560), (2592, 64)])
+def test_wide_forms(gpu_ctx, O, hidden, dim):
+    """The row lengths at which a wave's blocks per part, and the loads of a
+    stage, step up: 4 / 5, 8 / 9, 12 / 13, 16 / 17, 20 / 21 (two row tiles a step
+    below, odd numbers of them too), 24 / 25, 32 / 33, 40 / 41 blocks in one
+    part, 46, 48 / 49, 64 / 65, 80 / 81 in two; passes of two tiles and of one
+    entry."""
+    _layer_run(gpu_ctx, O, moe_batch_fixture(hidden, dim, 1, 1, 0, "normal"), 65)
