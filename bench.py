@@ -37,11 +37,11 @@ INT8_DENSE_TOPS = 5000.0     # MI355X dense int8 MFMA
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_mx_mfma_decode_b64_36layers.md")
 MFMA_PROFILE = os.path.join(ROOT, "profiles", "k_mx_wide_prefill_b512_hot.md")
 # policy of the library's default for the wide launches (spt_abi.hip:
-# kGemmMinGroup, kGemmMinSelections, kGemmMinGain, kGemvMinExperts;
-# spt_kernels.hip: the costs of a wide pass of one and of two tiles and of a
-# GEMV pass)
-GEMM_MIN_GROUP, GEMM_MIN_SELECTIONS, GEMM_MIN_GAIN, GEMV_MIN_EXPERTS = 5, 384, 200, 4
-WIDE_COST1, WIDE_COST2, GEMV_PASS_COST = 25, 37, 14
+# kGemmMinGroup, kGemmMinSelections, and at this shape the costs of
+# set_pass_costs: a GEMV pass over an expert, a wide pass of one and of two
+# tiles, the two launches of each kind, ns)
+GEMM_MIN_GROUP, GEMM_MIN_SELECTIONS = 5, 384
+GEMV_PASS_NS, WIDE_PASS_NS, GEMV_LAUNCH_NS, WIDE_LAUNCH_NS = 2100, (3750, 5550), 16000, 18000
 # selections per grouped-GEMV weight pass (spt_kernels.h: kGemvTokens)
 GEMV_TOKENS = 4
 # host threads for the CPU baseline: the host's CPU share per GPU
@@ -379,12 +379,13 @@ def prefill(args, ctx, dl, shp, W, stream, reps=20):
         c = counts.cpu().numpy()
         distinct = int(np.count_nonzero(c))
         n = B * k
-        big = c[c >= GEMM_MIN_GROUP]
-        rem = big % 64
-        wide = big // 64 * WIDE_COST2 + np.where(rem == 0, 0, np.where(rem > 32, WIDE_COST2, WIDE_COST1))
-        gain = int(np.sum((big + GEMV_TOKENS - 1) // GEMV_TOKENS * GEMV_PASS_COST - wide))
-        gemm_on = n >= GEMM_MIN_SELECTIONS and gain >= GEMM_MIN_GAIN and int(np.sum((big + 63) // 64)) * (D // 32) >= 512
-        gemm_min = 1 if int(np.sum((c > 0) & (c < GEMM_MIN_GROUP))) < GEMV_MIN_EXPERTS else GEMM_MIN_GROUP
+        rem = c % 64
+        wide = c // 64 * WIDE_PASS_NS[1] + np.where(rem == 0, 0, np.where(rem > 32, WIDE_PASS_NS[1], WIDE_PASS_NS[0]))
+        save = (c + GEMV_TOKENS - 1) // GEMV_TOKENS * GEMV_PASS_NS - wide
+        lose = -int(save[c < GEMM_MIN_GROUP].sum())
+        gain = int(save[c >= GEMM_MIN_GROUP].sum())
+        gemm_on = n >= GEMM_MIN_SELECTIONS and WIDE_LAUNCH_NS + min(lose, GEMV_LAUNCH_NS) - gain < GEMV_LAUNCH_NS
+        gemm_min = 1 if lose < GEMV_LAUNCH_NS else GEMM_MIN_GROUP
         big = c[c >= gemm_min]
         gemm_sel = int(big.sum()) if gemm_on else 0
         # warm for at least 60 ms of back-to-back layers: a few calls after

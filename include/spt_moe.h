@@ -130,8 +130,9 @@ int spt_ctx_set_cancel_flag(struct spt_ctx *ctx, const volatile int32_t *flag);
 /* Expert groups of at least min_group selections run through the grouped
  * GEMM (block-scaled MFMA, up to 64 selections per pass over the expert's
  * weights); smaller groups through the grouped GEMV (4 per pass).  0 restores
- * the default policy: groups of 5 or more when the batch holds at least 384
- * selections and the passes saved outweigh the launches.  Results are the
+ * the default policy: in batches of at least 384 selections, the cheapest by
+ * estimate of the GEMV alone, the GEMM for groups of 5 or more beside it, and
+ * the GEMM alone; below, the GEMV.  Results are the
  * same either way within the fp32 tolerance (the per-block sums are exact on
  * both).  No reference counterpart: the reference picks its CPU loop by tile
  * size (forward/mxfp4_batch.go:55-95). */

@@ -396,24 +396,39 @@ int copy_tap(spt_ctx *ctx, void *dst, const void *src, size_t bytes) {
     return SPT_OK;
 }
 
-// Default policy for the wide product (spt_mx_wide.hip; measured on MI355X
-// with GPT-OSS shapes, us per layer): a group of one GEMV pass (up to four
-// selections) stays on the GEMV, which streams weights faster; larger groups
-// go to the wide launches, which read an expert's weights once per 64
-// selections, when the batch holds at least kGemmMinSelections selections and
-// the passes saved are worth more than the two launches (kGemmMinGain, about
-// 20 us of gate/up) and make two units or more for each workgroup.  GEMV only / thresholds of 9 / 5: uniform routing 96
-// tokens 354 / 363 / 359, 128: 436 / 432 / 414, 256: 721 / 567 / 536; Zipf(1.1)
-// 96: 284 / 207 / 204, 256: 654 / 309 / 307.  Below 384 selections the wide
-// launches' fixed cost outweighs the passes they save (Zipf(0.6): 48 tokens
-// 204 / 231 / 229, 64: 240 / 256 / 254).  With fewer than kGemvMinExperts
-// small groups these go to the wide launches too: a GEMV launch for a few
-// experts costs more than their share of the wide ones (uniform, 512 tokens:
-// 592 with five experts on the GEMV, 569 without).
+// Default policy for the wide product (spt_mx_wide.hip): batches of at least
+// kGemmMinSelections selections (below, its launches' fixed cost outweighs the
+// passes they save: Zipf(0.6) at GPT-OSS-120B shape, us a layer, GEMV only /
+// wide from five selections: 48 tokens 204 / 229, 64: 240 / 254) run their
+// groups by whichever is estimated the cheapest: the GEMV alone, the GEMV for
+// groups of one pass (up to four selections; it streams weights faster) and the
+// wide launches, which read an expert's weights once per 64 selections, for the
+// others, or the wide launches alone.  The estimate, from measured launches of
+// groups of 2 to 64 at widths from 512 to 2,880: a GEMV pass over an expert's
+// gate and up at 2,880 x 2,880 costs 1.4 us of the whole device, a wide pass of
+// one and of two tiles 2.5 and 3.7 (1.7 and 2.7 with two row tiles a step), in
+// proportion to the weights of a launch; and the GEMV's two launches 16 us, the
+// wide ones 18.  Over 1,638 layers (13 widths, 8 to 128 experts, 48 to 1,000
+// tokens, uniform to Zipf(1.1)) the choice takes 0.2 % more time than the best
+// of the three, at worst 14 %; one gain threshold for all widths took 19 %, at
+// worst 4.5 times.  At 2,880 wide, uniform, GEMV only / both: 96 tokens 354 / 359,
+// 128: 436 / 414, 256: 721 / 536.
 constexpr int kGemmMinGroup = 5;
 constexpr int kGemmMinSelections = 384;
-constexpr int kGemmMinGain = 200;
-constexpr int kGemvMinExperts = 4;
+constexpr int kGemvLaunchNs = 16000, kWideLaunchNs = 18000;
+
+// The estimate's costs of one layer.
+void set_pass_costs(spt::SelectOut &so, int64_t h, int64_t d) {
+    constexpr int64_t kTenth = 100, kUnit = 2 * 2880 * 90;  // blocks of gate and up of the measured expert
+    const int64_t gate_up = 2 * d * (h / 32), down = h * (d / 32);
+    auto cost = [&](int64_t nb, int wide, int narrow) { return spt::mx_wide_unit_rows((int)nb) > spt::kWideRows ? narrow : wide; };
+    so.gemv_cost = (int32_t)((gate_up + down) * 14 * kTenth / kUnit);
+    so.wide_cost[0] = (int32_t)((gate_up * cost(h / 32, 25, 17) + down * cost(d / 32, 25, 17)) * kTenth / kUnit);
+    so.wide_cost[1] = (int32_t)((gate_up * cost(h / 32, 37, 27) + down * cost(d / 32, 37, 27)) * kTenth / kUnit);
+    so.gemv_launch = kGemvLaunchNs;
+    so.wide_launch = kWideLaunchNs;
+}
+
 // Batches of up to this many selections (topk <= 4, no GEMM group) take the
 // decode path: top-k inside the gate/up launch, combine inside the down
 // launch, a workgroup per selection (spt_mx_decode.hip).  Measured on the
@@ -496,9 +511,8 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     so.active = (int32_t *)(S + L.o_act_list);
     so.n_active = (int32_t *)(S + L.o_na);
     so.gemm_min = use_gemm ? gemm_min : INT_MAX;
-    so.gemm_min_gain = forced ? INT_MIN : kGemmMinGain;
-    so.gemm_min_units = forced ? 0 : 2 * ctx->n_cu;
-    so.gv_min_experts = forced ? 0 : kGemvMinExperts;
+    so.by_cost = use_gemm && !forced;
+    set_pass_costs(so, h, d);
     so.gv_active = (int32_t *)(S + L.o_gv);
     so.gv_n = (int32_t *)(S + L.o_gvn);
     so.gv_pass_off = (int32_t *)(S + L.o_gvp);

@@ -33,14 +33,12 @@ struct SelectOut {
     // Experts with count >= gemm_min go to the wide launches, the others to
     // the grouped GEMV, each with its own packed expert list:
     int32_t gemm_min;
-    // ...provided they gain at least gemm_min_gain over the GEMV's passes (in
-    // the units of wide_cost and kGemvPassCost) and hold at least gemm_min_units
-    // units (passes x wide_units[0]: enough to fill the device); otherwise every
-    // expert goes to the GEMV.
-    int32_t gemm_min_gain, gemm_min_units;
-    // With fewer than gv_min_experts experts below gemm_min, those go to the
-    // wide launches too.
-    int32_t gv_min_experts;
+    // ...or, with by_cost, all of them to the one or to the other where that is
+    // cheaper (nanoseconds a layer): gemv_cost and wide_cost[0 / 1] a pass of an
+    // expert (wide: of up to 32 entries and of more), gemv_launch and wide_launch
+    // the two launches of a kind.
+    bool by_cost;
+    int32_t gemv_cost, wide_cost[2], gemv_launch, wide_launch;
     int32_t *gv_active;    // [E] GEMV experts, ascending
     int32_t *gv_n;
     int32_t *gv_pass_off;  // [E+1] prefix over GEMV experts of ceil(count / kGemvTokens)

@@ -180,14 +180,14 @@ constexpr int kSelWaves = kSelWG / 64;
 constexpr int kExpertBits = 8;
 static_assert(kMaxExperts <= 1 << kExpertBits, "expert ids");
 
-// Cost of a unit of a wide pass with one and with two 32-entry tiles, of a
-// unit of all passes over a list of c entries, and of the same rows in a GEMV
-// pass: tenths of a microsecond per expert on the whole device, gate/up at
-// GPT-OSS-120B shape (2.5, 3.7; GEMV 1.4).
-constexpr int kWideCost1 = 25, kWideCost2 = 37, kGemvPassCost = 14;
-__device__ inline int wide_cost(int c) {
+// Shares of a wide pass with one and with two 32-entry tiles (2.5 and 3.7 us
+// per expert on the whole device, gate/up at GPT-OSS-120B shape; 1.35 to 1.6
+// times as much for two at other widths), by which the launches deal their work.
+constexpr int kWideCost1 = 25, kWideCost2 = 37;
+// The cost of all passes over a list of c entries.
+__device__ inline int wide_cost(int c, int cost1 = kWideCost1, int cost2 = kWideCost2) {
     const int full = c / kGemmTokens, rem = c % kGemmTokens;
-    return full * kWideCost2 + (rem == 0 ? 0 : rem > 32 ? kWideCost2 : kWideCost1);
+    return full * cost2 + (rem == 0 ? 0 : rem > 32 ? cost2 : cost1);
 }
 
 // Last i < n with v[i] <= x, v ascending and v[0] <= x (0 for n = 0).
@@ -240,17 +240,23 @@ __device__ void pack_lists(int n, int E, const SelectOut &o, const int32_t *s_id
         // order; the number of the wide launches' experts and passes (ordered below)
         int pos = 0, na = 0, nv = 0, nm = 0, npass = 0, ntile = 0;
         const uint64_t below = (1ull << tid) - 1ull;
-        // what the wide passes over the threshold's experts would save, and the
-        // experts below it
-        int gain = 0, small = 0, passes = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int c = e0 + tid < E ? s_cnt[e0 + tid] : 0;
-            small += __builtin_popcountll(__ballot(c > 0 && c < o.gemm_min));
-            gain += lane63(wave_incl_scan((c > 0 && c >= o.gemm_min) ? (c + kGemvTokens - 1) / kGemvTokens * kGemvPassCost - wide_cost(c) : 0));
-            passes += lane63(wave_incl_scan((c > 0 && c >= o.gemm_min) ? (c + kGemmTokens - 1) / kGemmTokens : 0));
+        // the threshold, or the cheapest of three: the GEMV alone, both, the wide
+        // launches alone
+        bool gemm_on = true;
+        int gm_min = o.gemm_min;
+        if (o.by_cost) {
+            int save = 0, lose = 0;  // by wide passes over the experts at the threshold, and below it
+            for (int e0 = 0; e0 < E; e0 += 64) {
+                const int c = e0 + tid < E ? s_cnt[e0 + tid] : 0;
+                const int diff = (c + kGemvTokens - 1) / kGemvTokens * o.gemv_cost - wide_cost(c, o.wide_cost[0], o.wide_cost[1]);
+                if (c >= gm_min) save += diff;
+                else lose -= diff;
+            }
+            save = lane63(wave_incl_scan(save));
+            lose = lane63(wave_incl_scan(lose));
+            gemm_on = o.wide_launch + min(lose, o.gemv_launch) - save < o.gemv_launch;
+            if (lose < o.gemv_launch) gm_min = 1;
         }
-        const bool gemm_on = gain >= o.gemm_min_gain && (int64_t)passes * o.wide_units[0] >= o.gemm_min_units;
-        const int gm_min = gemm_on && small < o.gv_min_experts ? 1 : o.gemm_min;
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int e = e0 + tid;
             const int c = e < E ? s_cnt[e] : 0;

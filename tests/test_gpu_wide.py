@@ -122,3 +122,50 @@ def test_wide_forms(gpu_ctx, O, hidden, dim):
     part, 46, 48 / 49, 64 / 65, 80 / 81 in two; passes of two tiles and of one
     entry."""
     _layer_run(gpu_ctx, O, moe_batch_fixture(hidden, dim, 1, 1, 0, "normal"), 65)
+
+
+@pytest.mark.parametrize("hidden,experts,small,batch,route", [
+    (64, 128, 0, 192, "gemv"), (1536, 128, 0, 128, "gemv both"), (2880, 24, 12, 128, "both"),
+    (512, 8, 0, 200, "both wide"), (2880, 24, 8, 128, "wide")])
+def test_default_route(gpu_ctx, hidden, experts, small, batch, route):
+    """The default policy's three choices, told apart by their bits (the GEMV and
+    the wide product add the blocks in different orders): a narrow layer, and one
+    of four selections an expert, on the GEMV alone; large groups beside twelve
+    of three selections on both; large groups alone, or beside eight such (less
+    than the GEMV's own launches), on the wide product alone.  (With no group on
+    one side of the threshold two settings are the same.)"""
+    import torch
+
+    import spt
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(hidden + small)
+    lw = spt.MoELayer()
+    keep = [torch.randn(experts * hidden, generator=g, device="cuda") * 0.02]
+    lw.ffn_gate_inp = spt.Tensor.make("router", spt.TYPE_F32, [hidden, experts], keep[0].data_ptr(), experts * hidden * 4)
+    for name in ("gate", "up", "down"):
+        w = torch.randint(0, 256, (experts * hidden * hidden // 32, 17), generator=g, device="cuda", dtype=torch.uint8)
+        w[:, 0] = 118 + w[:, 0] % 7
+        keep.append(w)
+        setattr(lw, f"ffn_{name}_exps", spt.Tensor.make(name, spt.TYPE_MXFP4, [hidden, hidden, experts], w.data_ptr(), w.numel()))
+    cfg = spt.MoEConfig(hidden, hidden, experts, 4)
+    t = torch.arange(batch, device="cuda")
+    large = experts - small
+    logits = torch.zeros(batch, experts, device="cuda")
+    for j in range(4):
+        e = (4 * t + j) % large
+        if j == 0 and small:  # three tokens each for the last `small` experts
+            e = torch.where(t < 3 * small, large + t % small, e)
+        logits[t, e] = 1.0 + j
+    x = torch.randn(batch * hidden, generator=g, device="cuda")
+    outs = {}
+    try:
+        for name, threshold in (("default", 0), ("gemv", 1 << 30), ("both", 5), ("wide", 1)):
+            gpu_ctx.set_gemm_min_group(threshold)
+            outs[name] = torch.empty(batch * hidden, device="cuda")
+            gpu_ctx.forward_moe_batch(cfg, lw, x, outs[name], batch, spt.make_taps(logits_in=logits))
+            torch.cuda.synchronize()
+    finally:
+        gpu_ctx.set_gemm_min_group(0)
+    same = [n for n in ("gemv", "both", "wide") if torch.equal(outs["default"].view(torch.int32), outs[n].view(torch.int32))]
+    assert same == route.split()
