@@ -418,13 +418,13 @@ constexpr int kGemmMinSelections = 384;
 constexpr int kGemvLaunchNs = 16000, kWideLaunchNs = 18000;
 
 // The estimate's costs of one layer.
-void set_pass_costs(spt::SelectOut &so, int64_t h, int64_t d) {
+void set_pass_costs(spt::SelectOut &so, int64_t h, int64_t d, const int unit_rows[2]) {
     constexpr int64_t kTenth = 100, kUnit = 2 * 2880 * 90;  // blocks of gate and up of the measured expert
     const int64_t gate_up = 2 * d * (h / 32), down = h * (d / 32);
-    auto cost = [&](int64_t nb, int wide, int narrow) { return spt::mx_wide_unit_rows((int)nb) > spt::kWideRows ? narrow : wide; };
+    auto cost = [&](int l, int wide, int narrow) { return unit_rows[l] > spt::kWideRows ? narrow : wide; };
     so.gemv_cost = (int32_t)((gate_up + down) * 14 * kTenth / kUnit);
-    so.wide_cost[0] = (int32_t)((gate_up * cost(h / 32, 25, 17) + down * cost(d / 32, 25, 17)) * kTenth / kUnit);
-    so.wide_cost[1] = (int32_t)((gate_up * cost(h / 32, 37, 27) + down * cost(d / 32, 37, 27)) * kTenth / kUnit);
+    so.wide_cost[0] = (int32_t)((gate_up * cost(0, 25, 17) + down * cost(1, 25, 17)) * kTenth / kUnit);
+    so.wide_cost[1] = (int32_t)((gate_up * cost(0, 37, 27) + down * cost(1, 37, 27)) * kTenth / kUnit);
     so.gemv_launch = kGemvLaunchNs;
     so.wide_launch = kWideLaunchNs;
 }
@@ -512,17 +512,20 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
     so.n_active = (int32_t *)(S + L.o_na);
     so.gemm_min = use_gemm ? gemm_min : INT_MAX;
     so.by_cost = use_gemm && !forced;
-    set_pass_costs(so, h, d);
     so.gv_active = (int32_t *)(S + L.o_gv);
     so.gv_n = (int32_t *)(S + L.o_gvn);
     so.gv_pass_off = (int32_t *)(S + L.o_gvp);
     so.gm_active = (int32_t *)(S + L.o_gm);
+    int unit_rows[2] = {0, 0};  // of the two wide launches
     if (use_gemm) {
         so.gm_start = (int32_t *)(S + L.o_gms);
         so.gm_grid = spt::mx_wide_grid();
-        const int64_t gate_up = spt::mx_wide_unit_rows((int)nbh), down = spt::mx_wide_unit_rows((int)nbd);
-        so.wide_units[0] = (int32_t)((d + gate_up - 1) / gate_up);
-        so.wide_units[1] = (int32_t)((h + down - 1) / down);
+        const int passes = (int)std::max(std::min(n, E), n / spt::kGemmTokens);  // with every expert in use
+        unit_rows[0] = spt::mx_wide_unit_rows((int)nbh, (int)d, passes);
+        unit_rows[1] = spt::mx_wide_unit_rows((int)nbd, (int)h, passes);
+        so.wide_units[0] = (int32_t)((d + unit_rows[0] - 1) / unit_rows[0]);
+        so.wide_units[1] = (int32_t)((h + unit_rows[1] - 1) / unit_rows[1]);
+        set_pass_costs(so, h, d, unit_rows);
     }
     // the two grouped GEMV launches' start table, for their grids
     const int slots = (int)(n < E ? n : E);
@@ -672,6 +675,7 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
         gg.w[1] = ga.w[1];
         gg.expert_bytes = ga.expert_bytes;
         gg.rows = ga.rows;
+        gg.unit_rows = unit_rows[0];
         gg.nb = ga.nb;
         for (int i = 0; i < 2; i++) {
             gg.bias[i] = ga.bias[i];
@@ -721,6 +725,7 @@ int run_moe_at(spt_ctx *ctx, const spt_moe_layer *lw, const float *x, float *out
         gd.w[0] = da.w[0];
         gd.expert_bytes = da.expert_bytes;
         gd.rows = da.rows;
+        gd.unit_rows = unit_rows[1];
         gd.nb = da.nb;
         gd.bias[0] = da.bias[0];
         gd.bias_bytes[0] = da.bias_bytes[0];

@@ -164,6 +164,7 @@ struct MxWideArgs {
     int8_t *act_codes;
     uint8_t *act_tab;
     uint8_t *act_blocks34;
+    int unit_rows;           // rows of a unit: kWideRows or twice that (mx_wide_unit_rows); the launch's, not read by the kernel
 };
 
 // One more Q4_0 matrix of a GEMV launch over several projections of the
@@ -282,9 +283,10 @@ hipError_t launch_mx_mfma(hipStream_t s, GemvMode mode, const MxMfmaArgs &a, int
 // The grid launch_mx_mfma uses for these arguments (0: nothing to launch).
 int mx_mfma_grid(GemvMode mode, const MxMfmaArgs &a, int slots);
 // The grid of launch_mx_wide (SelectOut::gm_grid), and the output rows of its
-// units for an input of nb blocks (SelectOut::wide_units).
+// units (MxWideArgs::unit_rows, SelectOut::wide_units) over at least `passes`
+// passes.
 int mx_wide_grid();
-int mx_wide_unit_rows(int nb);
+int mx_wide_unit_rows(int nb, int rows, int passes);
 // Whether the wide launches take expert matrices of this many bytes (their
 // loads use offsets past 2^31 for "nothing").
 inline bool mx_wide_fits(uint64_t expert_bytes) { return expert_bytes <= 0x7FFFFF00ull; }

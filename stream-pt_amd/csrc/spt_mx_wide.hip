@@ -52,11 +52,12 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kStages = 3;
-constexpr int kMaxPart = 45;         // blocks of a row per stage
-constexpr int kMaxQuarter = 20;      // the same with two row tiles a step
+// Blocks of a row per stage, as the LDS allows: half a row, a whole row, a whole
+// row of each of two row tiles.
+constexpr int kMaxHalf = 45, kMaxRow = 48, kMaxRow2 = 24;
 constexpr int kLoadWaves = 4;        // waves that issue the loads (one per SIMD)
 constexpr int kPartsLds = kWaves * kWideRows * kGemmTokens * 4;  // the waves' partial sums of a step
-constexpr int kStaticLds = 20 * 1024;  // static LDS of a workgroup, at most
+constexpr int kStaticLds1 = 11 * 1024, kStaticLds2 = 19 * 1024;  // static LDS of a workgroup, rows in one part and in two
 constexpr int kDownStores = 1, kActStores = 4;  // vector stores of an epilogue that stores (down; up step)
 constexpr int kBiasWave = kLoadWaves - 1;  // loads the biases
 constexpr int kEMin = 4, kEMax = 240;
@@ -81,12 +82,13 @@ __host__ __device__ constexpr int wave_loads(int blocks) { return (stage_loads<R
 // the 32 lanes' reads meet no bank twice.
 __device__ inline int slot_row(int p) { return (p & 16) == 0 ? p : (p & ~15) + ((p + 1) & 15); }
 __device__ inline int row_slot(int r) { return r < 16 ? r : 16 + ((r - 1) & 15); }
-static_assert(2 * kMaxPart >= kMxMaxInput / 32, "a row is at most two parts");
+static_assert(2 * kMaxHalf >= kMxMaxInput / 32, "a row is at most two parts");
 // dynamic LDS of a workgroup: the stages and the waves' partial sums
 template <int RT>
 constexpr int dynamic_lds(int blocks) { return kStages * 1024 * stage_loads<RT>(blocks) + kPartsLds; }
-static_assert(dynamic_lds<1>(kMaxPart) + kStaticLds <= 160 * 1024, "LDS");
-static_assert(dynamic_lds<2>(kMaxQuarter) + kStaticLds + 6 * 1024 <= 160 * 1024, "LDS with two row tiles");
+static_assert(dynamic_lds<1>(kMaxHalf) + kStaticLds2 <= 160 * 1024, "LDS, rows in two parts");
+static_assert(dynamic_lds<1>(kMaxRow) + kStaticLds1 <= 160 * 1024, "LDS, rows in one part");
+static_assert(dynamic_lds<2>(kMaxRow2) + kStaticLds1 <= 160 * 1024, "LDS, two row tiles");
 static_assert(kGemmTokens == 64, "two 32-entry tiles per pass");
 
 // Waits for a stage (the waves that load; the barrier after it does for the
@@ -205,7 +207,7 @@ __device__ float lut_dot(const ByteView &v, uint32_t row_pos, int nb, const int8
 // that: with RT = 2 four waves split K on the first 32 rows of a step, four on
 // the next (the last step's second tile may lie past the rows: its results go
 // nowhere).  Weights come by LDS DMA in stages of one part (half a row beyond
-// 45 blocks) of a step's rows -- a ring of three stages, two in flight while one
+// 48 blocks) of a step's rows -- a ring of three stages, two in flight while one
 // is multiplied; a row's part is contiguous in memory, so a stage is 32 or 64
 // runs of up to 765 bytes.
 //
@@ -218,13 +220,14 @@ template <int MODE, int P, int NJ, int RT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_mx_wide(MxWideArgs) {
     constexpr int kSub = MODE == kGateUp ? 2 : 1;  // steps per unit
     constexpr int KS = kWaves / RT, kStepRows = RT * kWideRows;  // parts of K; rows of a step
-    constexpr int kLoads = wave_loads<RT>(NJ * KS < kMaxPart ? NJ * KS : kMaxPart);
+    constexpr int kBlocks = P == 2 ? kMaxHalf : RT == 1 ? kMaxRow : kMaxRow2;
+    constexpr int kLoads = wave_loads<RT>(NJ * KS < kBlocks ? NJ * KS : kBlocks);
     static_assert(RT == 1 || P == 1, "rows in parts: one row tile");
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ uint32_t s_bias[8][64];      // raw bias dwords of a step's rows
     __shared__ int s_ent[2][kGemmTokens];   // per pass parity: list entries (-1 past the end)
     __shared__ uint32_t s_apos[kLoads][64 * kLoadWaves];  // each loading thread's offsets of a stage
-    __shared__ v4f s_gate[MODE == kGateUp ? RT * kThreads : 1];  // gate sums of a unit, for its up step
+    __shared__ v4f s_gate[MODE == kGateUp && P == 2 ? kThreads : 1];  // gate sums of a unit, for its up step
     __shared__ uint32_t s_spare[256];       // where the loads past a stage's go
     __shared__ uint32_t s_special[2][RT];   // per step parity and row tile: rows with special scales
 
@@ -458,6 +461,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     };
 
     // ---- the epilogue of the previous step ---------------------------------------
+    v4f gate_sums[RT];  // s_gate where registers are left (rows in one part; the LDS goes to longer stages)
     int q_u = 0, q_e = 0, q_sub = 0, q_par = 0, q_ntile = 0, q_step = 0;
     // NT tiles, row tile S: lane l of wave v takes TW = 4 NT entries' rows, R =
     // 2 NT rows each: entry TW * v + l % TW, rows R * (l / TW) .. + R - 1.
@@ -518,12 +522,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             return;
         }
         // (a gate sum is read back by the thread that wrote it, in the same pass)
-        vRf &gate = *reinterpret_cast<vRf *>(&s_gate[kThreads * S + 64 * wave + ln]);
+        v4f *const sg = &s_gate[P == 2 ? 64 * wave + ln : 0];
         if (q_sub == 0) {
-            gate = s;
+#pragma unroll
+            for (int i = 0; i < R; i++)
+                if (P == 1) gate_sums[S][i] = s[i];
+            if (P == 2) *reinterpret_cast<vRf *>(sg) = s;
             return;
         }
-        const vRf gv = gate;
+        vRf gv;
+#pragma unroll
+        for (int i = 0; i < R; i++) gv[i] = gate_sums[S][i];
+        if (P == 2) gv = *reinterpret_cast<const vRf *>(sg);
         vRf act;
         {
             float g[R], u[R], v[R];
@@ -710,55 +720,68 @@ template <int MODE, int P, int NJ, int RT>
 static hipError_t launch_wide_form(hipStream_t s, const MxWideArgs &a, int nb0) {
     // one-time opt-in to more than 64 KB of dynamic LDS
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mx_wide<MODE, P, NJ, RT>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       dynamic_lds<RT>(RT == 2 ? kMaxQuarter : kMaxPart));
+                                                       dynamic_lds<RT>(P == 2 ? kMaxHalf : RT == 1 ? kMaxRow : kMaxRow2));
     if (attr != hipSuccess) return attr;
     hipLaunchKernelGGL((k_mx_wide<MODE, P, NJ, RT>), dim3(mx_wide_grid()), dim3(kThreads), dynamic_lds<RT>(nb0), s, a);
     return hipGetLastError();
 }
 
 // Rows of a step of a launch over rows of nb blocks: two row tiles as long as
-// their stages fit the LDS.  A step's exchange of partial sums, its barriers and
-// the start of its loads cost about 4,000 cycles however short the rows are (at
-// 90 blocks the whole step is 10,000).  Gate/up of 128 experts, 12 entries each,
-// us, one tile / two: 512 inputs x 2,880 rows 189 / 149; down 2,880 inputs' 512:
-// 64 / 50; 512 x 512, six entries: 33.0 / 28.1.
-int mx_wide_unit_rows(int nb) { return nb <= kMaxQuarter ? 2 * kWideRows : kWideRows; }
+// their stages fit the LDS and there are five steps or more for a workgroup.  A
+// step's exchange of partial sums, its barriers and the start of its loads cost
+// about 4,000 cycles however short the rows are (at 90 blocks the whole step is
+// 10,000); with few steps the last one, twice as long, costs as much.  Us, one
+// tile / two: gate/up of 256 experts of 512 x 512, two entries each (8 steps a
+// workgroup) 74.9 / 58.1, 768 x 768 (12) 110 / 86.6; 128 experts, eight each, (4)
+// 40.6 / 32.8, (6) 58.6 / 47.6; 32 experts, 64 each, (1) 19.9 / 19.9, (1.5) 27.6 /
+// 31.1; layers of 768 x 768 with three to four steps 2 to 5 us the longer.
+// `passes` is a lower bound: the experts in use are not known here.
+int mx_wide_unit_rows(int nb, int rows, int passes) {
+    const int64_t steps = (int64_t)passes * ((rows + 2 * kWideRows - 1) / (2 * kWideRows));
+    return nb <= kMaxRow2 && steps >= 5 * mx_wide_grid() ? 2 * kWideRows : kWideRows;
+}
 
 // The form with exactly the blocks per wave and part of this row, rounded up:
 // a block past the part costs its products, a load past the stage's its issue
-// (1,536 inputs, 24 blocks a part, 128 experts: gate/up and down 162 + 77 us with
-// four blocks a wave and 28 loads a stage, 139 + 64 with three and 15).
+// (1,536 inputs, 128 experts, gate/up and down: 162 + 77 us in two parts with four
+// blocks a wave and 28 loads a stage, 139 + 64 with three and 15, 136 + 60 in one
+// part of six).
 template <int MODE>
 static hipError_t launch_wide_mode(hipStream_t s, const MxWideArgs &a) {
-    if (a.nb <= kMaxQuarter) {
+    if (a.unit_rows == 2 * kWideRows) {
         switch ((a.nb + 3) / 4) {
         case 1:
         case 2: return launch_wide_form<MODE, 1, 2, 2>(s, a, a.nb);
         case 3: return launch_wide_form<MODE, 1, 3, 2>(s, a, a.nb);
         case 4: return launch_wide_form<MODE, 1, 4, 2>(s, a, a.nb);
-        default: return launch_wide_form<MODE, 1, 5, 2>(s, a, a.nb);
+        case 5: return launch_wide_form<MODE, 1, 5, 2>(s, a, a.nb);
+        default: return launch_wide_form<MODE, 1, 6, 2>(s, a, a.nb);
         }
     }
-    const int nb0 = a.nb <= kMaxPart ? a.nb : (a.nb + 1) / 2, nj = (nb0 + kWaves - 1) / kWaves;
-    if (a.nb <= kMaxPart) {
-        switch (nj) {
-        case 3: return launch_wide_form<MODE, 1, 3, 1>(s, a, nb0);
-        case 4: return launch_wide_form<MODE, 1, 4, 1>(s, a, nb0);
-        case 5: return launch_wide_form<MODE, 1, 5, 1>(s, a, nb0);
-        default: return launch_wide_form<MODE, 1, 6, 1>(s, a, nb0);
+    if (a.nb <= kMaxRow) {
+        switch ((a.nb + kWaves - 1) / kWaves) {
+        case 1:
+        case 2: return launch_wide_form<MODE, 1, 2, 1>(s, a, a.nb);
+        case 3: return launch_wide_form<MODE, 1, 3, 1>(s, a, a.nb);
+        case 4: return launch_wide_form<MODE, 1, 4, 1>(s, a, a.nb);
+        case 5: return launch_wide_form<MODE, 1, 5, 1>(s, a, a.nb);
+        default: return launch_wide_form<MODE, 1, 6, 1>(s, a, a.nb);
         }
     }
-    switch (nj) {
-    case 3: return launch_wide_form<MODE, 2, 3, 1>(s, a, nb0);
+    const int nb0 = (a.nb + 1) / 2;
+    switch ((nb0 + kWaves - 1) / kWaves) {
     case 4: return launch_wide_form<MODE, 2, 4, 1>(s, a, nb0);
     case 5: return launch_wide_form<MODE, 2, 5, 1>(s, a, nb0);
     default: return launch_wide_form<MODE, 2, 6, 1>(s, a, nb0);
     }
 }
+static_assert((kMaxRow + 2) / 2 > 3 * kWaves, "a half row is four blocks a wave or more");
 
 hipError_t launch_mx_wide(hipStream_t s, GemvMode mode, const MxWideArgs &a) {
     if (a.rows <= 0) return hipSuccess;
-    if (a.nb <= 0 || a.nb > 2 * kMaxPart || a.rows % kWideRows != 0 || !a.start || !mx_wide_fits(a.expert_bytes)) return hipErrorInvalidConfiguration;
+    if (a.nb <= 0 || a.nb > 2 * kMaxHalf || a.rows % kWideRows != 0 || !a.start || !mx_wide_fits(a.expert_bytes) ||
+        (a.unit_rows != kWideRows && (a.unit_rows != 2 * kWideRows || a.nb > kMaxRow2)))
+        return hipErrorInvalidConfiguration;
     if (mode == kGateUp) return launch_wide_mode<kGateUp>(s, a);
     if (mode == kDown) return launch_wide_mode<kDown>(s, a);
     return hipErrorInvalidValue;

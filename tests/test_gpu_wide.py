@@ -112,16 +112,40 @@ def test_route_wide_bits(gpu_ctx, O, hidden, experts, batch):
     assert np.array_equal(bits(got.reshape(-1)), bits(np.asarray(want, np.float32).reshape(-1)))
 
 
-@pytest.mark.parametrize("hidden,dim", [(128, 160), (256, 288), (384, 416), (512, 544), (640, 672),
-                                        (768, 800), (1024, 1056), (1280, 1312),
-                                        (1472, 1536), (1568, 2048), (2080, 2560), (2592, 64)])
+@pytest.mark.parametrize("hidden,dim", [(256, 512), (768, 800), (1024, 1056), (1280, 1312), (1472, 1536), (1568, 2048),
+                                        (2080, 2560), (2592, 64)])
 def test_wide_forms(gpu_ctx, O, hidden, dim):
     """The row lengths at which a wave's blocks per part, and the loads of a
-    stage, step up: 4 / 5, 8 / 9, 12 / 13, 16 / 17, 20 / 21 (two row tiles a step
-    below, odd numbers of them too), 24 / 25, 32 / 33, 40 / 41 blocks in one
-    part, 46, 48 / 49, 64 / 65, 80 / 81 in two; passes of two tiles and of one
-    entry."""
+    stage, step up: 8, 16, 24 / 25, 32 / 33, 40 / 41, 46 / 48 blocks in one part,
+    49, 64 / 65, 80 / 81 in two; passes of two tiles and of one entry."""
     _layer_run(gpu_ctx, O, moe_batch_fixture(hidden, dim, 1, 1, 0, "normal"), 65)
+
+
+@pytest.mark.parametrize("hidden,dim", [(256, 320), (320, 288), (352, 320), (384, 416), (512, 288), (544, 320), (640, 288),
+                                        (672, 320), (768, 288), (288, 768)])
+def test_wide_two_row_tiles(gpu_ctx, O, hidden, dim):
+    """Steps of two row tiles (256 experts of five steps and more): blocks a wave
+    stepping up at 8 / 9, 12 / 13, 16 / 17, 20 / 21 and 24, odd numbers of row
+    tiles; groups of 65 entries (two tiles, then one entry), 40, and one each;
+    scales outside the MFMA's range in either tile."""
+    from test_gpu_moe import _run, check_stagewise, gemm_path
+
+    lay = moe_batch_fixture(hidden, dim, 256, 1, 0, "normal")
+    for name, rows, nb in (("gate", dim, hidden // 32), ("up", dim, hidden // 32), ("down", hidden, dim // 32)):
+        w = lay[name] = lay[name].copy()
+        w = w.reshape(256, rows, nb, 17)
+        w[5, 3, 0, 0] = 255
+        w[5, 41, nb - 1, 0] = 3
+        w[9, rows - 2, nb // 2, 0] = 241
+    keep, cfg, lw = device_moe_layer(lay)
+    batch = 136
+    x = moe_batch_x(batch, hidden, "normal")
+    logits = np.zeros((batch, 256), np.float32)
+    expert = np.r_[np.full(65, 5), np.full(40, 9), np.arange(20, 51)]
+    logits[np.arange(batch), expert] = 1.0
+    with gemm_path(gpu_ctx, "gemm"):
+        g = _run(gpu_ctx, cfg, lw, x, batch, logits.reshape(-1))
+    check_stagewise(O, lay, x, batch, g, logits, sample=[0, 1, 31, 32, 63, 64, 65, 96, 97, 104, 105, 135])
 
 
 @pytest.mark.parametrize("hidden,experts,small,batch,route", [
