@@ -288,9 +288,14 @@ int mx_mfma_grid(GemvMode mode, const MxMfmaArgs &a, int slots);
 int mx_wide_grid();
 int mx_wide_unit_rows(int nb, int rows, int passes);
 // Whether the wide launches take expert matrices of this many bytes (their
-// loads use offsets past 2^31 for "nothing").
-inline bool mx_wide_fits(uint64_t expert_bytes) { return expert_bytes <= 0x7FFFFF00ull; }
+// loads use offsets past 2^31 for "nothing"): those of every layer within
+// kMxMaxInput, the output of one projection being the input of the other.
+constexpr bool mx_wide_fits(uint64_t expert_bytes) { return expert_bytes <= 0x7FFFFF00ull; }
+static_assert(mx_wide_fits((uint64_t)(kMxMaxInput / 32 * 17) * kMxMaxInput), "the widest experts");
 hipError_t launch_mx_wide(hipStream_t s, GemvMode mode, const MxWideArgs &a);
+// nbytes of elements of `width` (2 or 4) bytes that begin at any address,
+// copied to an aligned one.
+hipError_t launch_align_elements(hipStream_t s, const void *src, uint64_t nbytes, int width, void *dst);
 // Q4_0 x Q8_0 for a batch: the int8-MFMA GEMM (spt_q40_gemm.hip, tiles of
 // kQ40TileRows rows x kQ40TileTokens tokens) from kQ40GemmMinTokens tokens
 // on kQ40GemmMinRows output rows and more, and from kQ40SplitMinTokens

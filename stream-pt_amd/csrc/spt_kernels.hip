@@ -116,6 +116,31 @@ hipError_t launch_quantize(hipStream_t s, const float *x, int64_t nblocks, int8_
     return hipGetLastError();
 }
 
+// (Biases that begin between elements: 1.5 MB of F32 at GPT-OSS-120B shape.  The
+// wide product reads them by DMA in whole dwords; a path for others in its
+// epilogue cost it 1 to 3 % where it is not taken.)
+__global__ __launch_bounds__(kWG) void k_align_elements(const uint8_t *__restrict__ src, uint64_t n, int width, uint8_t *__restrict__ dst) {
+    const uint64_t i = (uint64_t)blockIdx.x * kWG + threadIdx.x;
+    if (i >= n) return;
+    if (width == 4) {
+        uint32_t v;
+        __builtin_memcpy(&v, src + 4 * i, 4);
+        reinterpret_cast<uint32_t *>(dst)[i] = v;
+    } else {
+        uint16_t v;
+        __builtin_memcpy(&v, src + 2 * i, 2);
+        reinterpret_cast<uint16_t *>(dst)[i] = v;
+    }
+}
+
+hipError_t launch_align_elements(hipStream_t s, const void *src, uint64_t nbytes, int width, void *dst) {
+    const uint64_t n = nbytes / (uint64_t)width;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_align_elements, dim3((unsigned)((n + kWG - 1) / kWG)), dim3(kWG), 0, s, static_cast<const uint8_t *>(src), n, width,
+                       static_cast<uint8_t *>(dst));
+    return hipGetLastError();
+}
+
 hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, bool gemm,
                             int8_t *codes, float *scales, int32_t *sumq) {
     if (nblocks <= 0) return hipSuccess;

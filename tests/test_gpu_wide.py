@@ -193,3 +193,43 @@ def test_default_route(gpu_ctx, hidden, experts, small, batch, route):
         gpu_ctx.set_gemm_min_group(0)
     same = [n for n in ("gemv", "both", "wide") if torch.equal(outs["default"].view(torch.int32), outs[n].view(torch.int32))]
     assert same == route.split()
+
+
+@pytest.mark.parametrize("bias,off", [(0, 1), (0, 2), (0, 3), (1, 1), (30, 1)])
+@pytest.mark.parametrize("form", ["arena", "noalloc"])
+def test_wide_biases_between_elements(gpu_ctx, O, bias, off, form):
+    """Expert biases that begin between elements give a forced wide product the
+    same bits as aligned ones (and not the GEMV's, whose sums differ)."""
+    import torch
+
+    import spt
+    from test_gpu_moe import gemm_path
+
+    lay = moe_batch_fixture(768, 800, 3, 2, bias, "normal")
+    keep, cfg, lw = device_moe_layer(lay)
+    batch = 70
+    x = torch.from_numpy(moe_batch_x(batch, 768, "normal")).cuda()
+
+    def run(path):
+        out = torch.full((batch * 768,), 9.0, device="cuda")
+        with gemm_path(gpu_ctx, path):
+            if form == "arena":
+                gpu_ctx.forward_moe_batch(cfg, lw, x, out, batch)
+            else:
+                from test_zz_no_alloc import _noalloc
+
+                assert _noalloc(gpu_ctx, cfg, lw, x, out, batch) == spt.OK
+            torch.cuda.synchronize()
+        return bits(out.cpu().numpy())
+
+    want, gemv = run("gemm"), run("gemv")
+    assert not np.array_equal(want, gemv)
+    for name in ("gate_bias", "up_bias", "down_bias"):
+        field = f"ffn_{name.split('_')[0]}_exps_bias"
+        t = getattr(lw, field)
+        buf = torch.zeros(t.nbytes + 8, dtype=torch.uint8, device="cuda")
+        buf[off:off + t.nbytes] = keep[name].view(torch.uint8)
+        keep["moved " + name] = buf
+        shape = [t.shape[i] for i in range(t.n_dims)]
+        setattr(lw, field, spt.Tensor.make(name, bias, shape, buf.data_ptr() + off, t.nbytes))
+    assert np.array_equal(run("gemm"), want) and np.array_equal(run("gemv"), gemv)
