@@ -929,20 +929,16 @@ struct Q40Proj {
     float *resid;
 };
 
-// The int8-MFMA GEMM forms and their split-K subset: spt::q40_gemm_form
-// and spt::q40_gemm_split (launch_q40_gemv's choice).
-bool q40_gemm_form(int64_t out, int64_t batch) { return spt::q40_gemm_form(out, batch); }
-bool q40_split(int64_t out, int64_t batch) { return spt::q40_gemm_split(out, batch); }
-
 // The launch of each of the np <= 3 projections of a call over one input:
 // 0 the GEMV, 1 the GEMM, 2 the split-K GEMM.
 void q40_launches(const Q40Proj *p, int np, int64_t batch, int *k) {
-    for (int i = 0; i < np; i++) k[i] = !q40_gemm_form(p[i].out, batch) ? 0 : !q40_split(p[i].out, batch) ? 1 : 2;
+    for (int i = 0; i < np; i++) k[i] = !spt::q40_gemm_form(batch) ? 0 : !spt::q40_gemm_split(p[i].out, batch) ? 1 : 2;
 }
 
 // Arena layout of a Q4_0 call over np projections sharing one input.  The
-// activation views (codes, widened scales, code sums) exist unless the input
-// is GGML Q8_0 blocks that every projection's GEMV reads directly.
+// activation views (codes, widened scales and, for the GEMV, code sums) exist
+// unless the input is GGML Q8_0 blocks that every projection's GEMV reads
+// directly.
 // A call of a few tokens (spt::q40_dec_form) runs as one launch that
 // quantizes or unpacks its input itself: no views.
 // A call of 5 to 64 tokens on inputs up to 128 blocks (spt::q40_tile_form)
@@ -956,28 +952,24 @@ struct Q40Plan {
 
 Q40Plan q40_plan(const Q40Proj *p, int np, int64_t nb, int64_t batch, bool q8_in, size_t base) {
     Q40Plan L{};
-    bool gemm = false;
     size_t part = 0;
     L.dec = spt::q40_dec_form(batch, nb);
     for (int i = 0; i < np; i++)
         if (p[i].w->nbytes >= spt::kQ40DecMaxBytes) L.dec = false;
     L.tile = !L.dec && spt::q40_tile_form(batch, nb);
+    L.gemm = !L.tile && spt::q40_gemm_form(batch);
     int k[3];
     q40_launches(p, np, batch, k);
-    for (int i = 0; i < np && !L.tile; i++) {
-        if (k[i] == 0) continue;
-        gemm = true;
+    for (int i = 0; i < np && L.gemm; i++)
         if (k[i] == 2) part += (size_t)spt::kQ40SplitK * batch * p[i].out * 4;
-    }
-    L.views = !L.dec && !L.tile && (!q8_in || gemm);
-    L.gemm = gemm;
+    L.views = !L.dec && !L.tile && (!q8_in || L.gemm);
     L.nb = nb;
     L.batch = batch;
     Carve c;
     c.off = base;
     L.o_c = c.take(L.views ? batch * nb * 32 : 0);
     L.o_s = c.take(L.views ? batch * nb * 4 : 0);
-    L.o_q = c.take(L.views ? batch * nb * 4 : 0);
+    L.o_q = c.take(L.views && !L.gemm ? batch * nb * 4 : 0);
     L.o_part = c.take(part);
     L.o_q34 = c.take(L.tile && !q8_in ? batch * nb * spt::kQ80Block : 0);
     L.total = c.off;
@@ -1038,10 +1030,10 @@ int run_q40_at(spt_ctx *ctx, const Q40Proj *p, int np, const Q40Plan &L, char *S
     }
     int8_t *codes = L.views ? (int8_t *)(S + L.o_c) : nullptr;
     float *scales = L.views ? (float *)(S + L.o_s) : nullptr;
-    int32_t *sumq = L.views ? (int32_t *)(S + L.o_q) : nullptr;
+    int32_t *sumq = L.views && !L.gemm ? (int32_t *)(S + L.o_q) : nullptr;
     if (L.views) {
         SPT_HIP(timed(ctx, SPT_KERNEL_QUANTIZE, [&] {
-            return spt::launch_q40_views(ctx->stream, x, xq34, batch * nb, L.gemm, codes, scales, sumq);
+            return spt::launch_q40_views(ctx->stream, x, xq34, batch * nb, codes, scales, sumq);
         }));
     }
     // the three launches' arguments: 0 GEMV, 1 wide GEMM, 2 split GEMM

@@ -297,28 +297,27 @@ hipError_t launch_mx_wide(hipStream_t s, GemvMode mode, const MxWideArgs &a);
 // copied to an aligned one.
 hipError_t launch_align_elements(hipStream_t s, const void *src, uint64_t nbytes, int width, void *dst);
 // Q4_0 x Q8_0 for a batch: the int8-MFMA GEMM (spt_q40_gemm.hip, tiles of
-// kQ40TileRows rows x kQ40TileTokens tokens) from kQ40GemmMinTokens tokens
-// on kQ40GemmMinRows output rows and more, and from kQ40SplitMinTokens
-// tokens on narrower projections; else the GEMV.  The GEMM splits K
+// kQ40TileRows rows x kQ40TileTokens tokens) from kQ40GemmMinTokens tokens;
+// else the GEMV.  The GEMM splits K
 // kQ40SplitK ways (partial sums in Q40Args::part, then summed in order,
 // when the caller provides the scratch) for projections of fewer than
 // kQ40SplitMaxTiles tiles (too few to fill the device); wider or longer ones
-// run unsplit, in the same launch as the others of their call (K and V of
-// 512 rows at 1,999 tokens: 55 us split and 12 us of reduction beside Q's 154,
-// against 40 more in Q's launch).
+// run unsplit, in the same launch as the others of their call.  The line is by
+// one matrix's tiles, so that a projection has the same bits alone and beside
+// others: one of 512 rows alone at 1,985 tokens, its first unsplit, 34.4 us (51.1
+// split), 960 rows 41.1 (72.9).  Beside Q, K and V of 512 rows would gain from
+// fewer tokens on (norm, Q/K/V and O, us, split / unsplit: 512 tokens 112.6 /
+// 115.8, 768: 174 / 155, 1,024: 192 / 180, 1,984: 336 / 310).
 // Unsplit, its sums are the GEMV's bit for bit; split, the partial sums of
 // the K ranges are added in range order (within rounding of the GEMV).
 constexpr int kQ40TileRows = 64;
 constexpr int kQ40TileTokens = 64;
 constexpr int kQ40GemmMinTokens = 32;
-constexpr int kQ40GemmMinRows = 1024;
 constexpr int kQ40SplitK = 4;
-constexpr int kQ40SplitMinTokens = 32;
 constexpr int kQ40SplitMaxTiles = 256;
-inline bool q40_gemm_form(int64_t rows, int64_t ntok) {
-    return (ntok >= kQ40GemmMinTokens && rows >= kQ40GemmMinRows) ||
-           (ntok >= kQ40SplitMinTokens && rows < kQ40GemmMinRows);
-}
+// By the tokens alone: the projections of a call share their input's views,
+// whose order of codes is the form's (q40_code_dword).
+inline bool q40_gemm_form(int64_t ntok) { return ntok >= kQ40GemmMinTokens; }
 inline bool q40_gemm_split(int64_t rows, int64_t ntok) {
     return ((rows + kQ40TileRows - 1) / kQ40TileRows) * ((ntok + kQ40TileTokens - 1) / kQ40TileTokens) <
            kQ40SplitMaxTiles;
@@ -342,11 +341,11 @@ constexpr int kQ40DecMaxNb = 128;
 constexpr uint64_t kQ40DecMaxBytes = 0x80000000ull;
 inline bool q40_dec_form(int64_t batch, int64_t nb) { return batch <= kQ40DecTokens && nb <= kQ40DecMaxNb; }
 hipError_t launch_q40_dec(hipStream_t s, const Q40Args &a);
-// The views of Q4_0 calls: codes (with `gemm` in the order of q40_code_dword),
-// widened scales and per-block code sums, for nblocks blocks of fp32 (x) or
-// GGML Q8_0 (blocks34) input.
-hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, bool gemm,
-                            int8_t *codes, float *scales, int32_t *sumq);
+// The views of Q4_0 calls for nblocks blocks of fp32 (x) or GGML Q8_0
+// (blocks34) input: widened scales and, of a GEMM call (sumq null), codes in the
+// order of q40_code_dword, else codes and per-block code sums.
+hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, int8_t *codes,
+                            float *scales, int32_t *sumq);
 hipError_t launch_q40_gemm(hipStream_t s, const Q40Args &a);
 // 5 to 64 tokens of inputs up to 128 blocks (spt_q40_tile.hip): a
 // workgroup per 16 output rows (when those workgroups all fit on the n_cu

@@ -59,16 +59,15 @@ __device__ __attribute__((always_inline)) inline uint32_t max8_bits(uint32_t m) 
     return m;
 }
 
-// The views the Q4_0 GEMM reads (codes, widened scales, code sums), from the
-// fp32 rows or from their GGML Q8_0 blocks: eight lanes per block, four
-// elements each (16-byte loads, 4-byte stores; x and the blocks need only
+// The views the Q4_0 GEMM reads (codes, widened scales) or the GEMV (code sums
+// too), from the fp32 rows or from their GGML Q8_0 blocks: eight lanes per block,
+// four elements each (16-byte loads, 4-byte stores; x and the blocks need only
 // their elements' alignment).  The arithmetic per element is
 // q8_quantize_half's.  Memory-bound: 8.2 M elements, 42 MB, from fp32 25.6 us
 // with a lane per element, from blocks (5.8 M, 12 MB) 15.0 us.
 template <bool Q8>
-__global__ __launch_bounds__(kWG) void k_q40_views(const void *__restrict__ in, int64_t nblocks, bool gemm,
-                                                   int8_t *__restrict__ codes, float *__restrict__ scales,
-                                                   int32_t *__restrict__ sumq) {
+__global__ __launch_bounds__(kWG) void k_q40_views(const void *__restrict__ in, int64_t nblocks, int8_t *__restrict__ codes,
+                                                   float *__restrict__ scales, int32_t *__restrict__ sumq) {
     const int tid = threadIdx.x, lane = tid & 63, i = tid & 7;
     const int64_t b = (int64_t)blockIdx.x * (kWG / 8) + (tid >> 3);
     const bool ok = b < nblocks;
@@ -98,12 +97,13 @@ __global__ __launch_bounds__(kWG) void k_q40_views(const void *__restrict__ in, 
 #pragma unroll
         for (int k = 0; k < 4; k++) w |= (uint32_t)(q8_code(v[k] * id) & 0xff) << (8 * k);
     }
-    const int s = sum8_int(__builtin_amdgcn_sdot4((int)w, 0x01010101, 0, false));
+    const bool gemm = !sumq;
+    const int s = gemm ? 0 : sum8_int(__builtin_amdgcn_sdot4((int)w, 0x01010101, 0, false));
     if (!ok) return;
     reinterpret_cast<uint32_t *>(codes)[b * 8 + (gemm ? q40_code_dword(i) : i)] = w;
     if (i == 0) {
         scales[b] = f16_bits_to_f32(dh);
-        sumq[b] = s;
+        if (!gemm) sumq[b] = s;
     }
 }
 
@@ -141,14 +141,14 @@ hipError_t launch_align_elements(hipStream_t s, const void *src, uint64_t nbytes
     return hipGetLastError();
 }
 
-hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, bool gemm,
-                            int8_t *codes, float *scales, int32_t *sumq) {
+hipError_t launch_q40_views(hipStream_t s, const float *x, const uint8_t *blocks34, int64_t nblocks, int8_t *codes,
+                            float *scales, int32_t *sumq) {
     if (nblocks <= 0) return hipSuccess;
     const dim3 grid((unsigned)((nblocks + kWG / 8 - 1) / (kWG / 8)));
     if (x)
-        hipLaunchKernelGGL(k_q40_views<false>, grid, dim3(kWG), 0, s, x, nblocks, gemm, codes, scales, sumq);
+        hipLaunchKernelGGL(k_q40_views<false>, grid, dim3(kWG), 0, s, x, nblocks, codes, scales, sumq);
     else
-        hipLaunchKernelGGL(k_q40_views<true>, grid, dim3(kWG), 0, s, blocks34, nblocks, gemm, codes, scales, sumq);
+        hipLaunchKernelGGL(k_q40_views<true>, grid, dim3(kWG), 0, s, blocks34, nblocks, codes, scales, sumq);
     return hipGetLastError();
 }
 
