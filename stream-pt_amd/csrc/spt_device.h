@@ -48,13 +48,10 @@ __device__ inline void dma16_nt(const u32x4v &rs, uint32_t lds, uint32_t voff, u
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds)
                  : "memory");
 }
-// dma16 without the memory clobber, for a load issued in the middle of the
+// dma16_nt without the memory clobber, for a load issued in the middle of the
 // reads of another stage: it writes only LDS that nothing reads before the
 // next full wait and barrier (which are memory clobbers themselves), so the
 // compiler may keep scheduling the surrounding LDS reads across it.
-__device__ inline void dma16_other_stage(const u32x4v &rs, uint32_t lds, uint32_t voff, uint32_t soff) {
-    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds));
-}
 __device__ inline void dma16_nt_other_stage(const u32x4v &rs, uint32_t lds, uint32_t voff, uint32_t soff) {
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds" ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds));
 }

@@ -1018,16 +1018,6 @@ static hipError_t launch_q40_maxp(hipStream_t s, const Q40Args &a) {
 
 hipError_t launch_q40_gemv(hipStream_t s, const Q40Args &a) {
     if (a.rows <= 0 || a.ntok <= 0) return hipSuccess;
-    if (a.nmore > 0 || a.xq34) {
-        // several matrices, or Q8_0 blocks in: the GEMV (the caller runs the
-        // GEMM forms one matrix at a time on unpacked activations)
-        const int per_lane = (a.nb + 15) / 16;
-        if (per_lane <= 1) return launch_q40_maxp<1>(s, a);
-        if (per_lane <= 2) return launch_q40_maxp<2>(s, a);
-        if (per_lane <= 4) return launch_q40_maxp<4>(s, a);
-        if (per_lane <= 6) return launch_q40_maxp<6>(s, a);
-        return launch_q40_maxp<8>(s, a);
-    }
     const int per_lane = (a.nb + 15) / 16;
     if (per_lane <= 1) return launch_q40_maxp<1>(s, a);
     if (per_lane <= 2) return launch_q40_maxp<2>(s, a);
