@@ -99,18 +99,6 @@ __device__ inline void load_block5(const ByteView &v, uint32_t pos, uint32_t d[5
     d[4] = __builtin_amdgcn_raw_buffer_load_b32(v.r, base + 16, 0, 0);
 }
 
-// The same five dwords when the caller already knows pos & 3.
-__device__ inline void load_block5_raw(const ByteView &v, uint32_t pos, uint32_t d[5]) {
-    uint32_t base = (pos + v.lead) & ~3u;
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 q = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(v.r, base, 0, 0));
-    d[0] = q.x;
-    d[1] = q.y;
-    d[2] = q.z;
-    d[3] = q.w;
-    d[4] = __builtin_amdgcn_raw_buffer_load_b32(v.r, base + 16, 0, 0);
-}
-
 // Workgroup barrier ordering LDS only: kernels whose waves communicate
 // through LDS alone use it in place of __syncthreads(), which would also wait
 // for every outstanding global load (draining the loads kept in flight).

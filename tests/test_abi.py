@@ -337,13 +337,13 @@ def test_forward_moe_unnamed_router_bias_still_checked(vctx):
 
 
 def test_moe_large_batches_run_as_slices(vctx):
-    """More than 4096 selections: the plain, host and Q8_0-input forms accept
+    """More than 8192 selections: the plain, host and Q8_0-input forms accept
     the batch (it runs as slices of whole tokens; the validation-only
-    context stops at the device), the tapped form refuses it, and the
-    experts-used and expert-count limits hold."""
+    context stops at the device).  More than 4096: the tapped form refuses it.
+    The experts-used and expert-count limits hold."""
     H, k = 32, 2
     cfg, lw = _moe_descriptors(H=H, k=k)
-    batch = 4096 // k + 1
+    batch = 8192 // k + 1
     n = batch * H
     assert _call_moe(vctx, cfg, lw, X, n, OUT, n, batch) == spt.ERR_DEVICE
     x = np.zeros(n, np.float32)
@@ -355,6 +355,8 @@ def test_moe_large_batches_run_as_slices(vctx):
                                             batch)
     assert rc == spt.ERR_DEVICE
     taps = spt.MoETaps()
+    batch = 4096 // k + 1
+    n = batch * H
     rc = spt.lib().spt_forward_moe_batch_ex(vctx.handle, C.byref(cfg), C.byref(lw), X, n, OUT, n, batch,
                                             C.byref(taps))
     assert rc == spt.ERR_INVALID and b"4096" in spt.lib().spt_last_error()

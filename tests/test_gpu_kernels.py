@@ -543,3 +543,38 @@ def test_q40_arena_of_a_layer(batch):
         torch.cuda.synchronize()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("batch", [1984, 1985, 1999])
+@pytest.mark.parametrize("kv", [512, 450])
+def test_q40_qkv_split_line(gpu_ctx, O, batch, kv):
+    """Narrow K and V beside Q on both sides of the split's line (256 tiles: 8 of
+    64 rows times 32 of 64 tokens, ragged in both): the fused call's bits are
+    those of each projection alone, and within tolerance the oracle's."""
+    import torch
+
+    import spt
+    from spt import synth
+
+    din = 288
+    assert spt_split(kv, 1984) and not spt_split(kv, 1985) and not spt_split(1088, batch)
+    x = synth.normal(synth.stream_key(3, batch), batch * din)
+    xd = torch.from_numpy(x).cuda()
+    keep, ws, ys, raw = [], [], [], []
+    for i, rows in enumerate((1088, kv, kv)):
+        w = synth.q40_bytes(synth.stream_key(20 + i, rows), rows, din)
+        raw.append(w)
+        keep.append(torch.from_numpy(w).cuda())
+        ws.append(spt.Tensor.make("w", spt.TYPE_Q4_0, [din, rows], keep[-1].data_ptr(), w.size))
+        ys.append(torch.full((batch * rows,), 9.0, device="cuda"))
+    gpu_ctx.mul_q40_qkv_batch_into(ws, None, xd, ys, batch)
+    for w, t, y in zip(raw, ws, ys):
+        alone = torch.full_like(y, 7.0)
+        gpu_ctx.mul_q40_batch_into(t, xd, alone, batch)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), alone.cpu().numpy().view(np.uint32))
+        rows = t.shape[1]
+        for lo, n in ((0, 70), (batch - 70, 70)):
+            assert_close(got[lo * rows:(lo + n) * rows], O.mul_q40_q8(w, np.ascontiguousarray(x[lo * din:(lo + n) * din]), din, rows, n),
+                         what="fused")

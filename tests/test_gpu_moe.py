@@ -403,14 +403,11 @@ def test_moe_output_any_alignment(gpu_ctx, O, batch):
     assert_close(a.cpu().numpy(), O.forward_moe_batch(lay, x, batch, q8=True), what="aligned output")
 
 
-def test_moe_gemm_side_stream_in_graph(O):
-    """With the grouped GEMM on (every group), a layer forks its GEMM
-    launches onto the context's second stream and joins them before the
-    combine.  Captured into a HIP graph on the context's stream and replayed
-    three times, with eager calls of another batch between the replays,
-    every replay's output equals the eager call's bit for bit (the fork and
-    the join are part of the graph), and the eager output matches the
-    oracle."""
+def test_moe_gemm_in_graph(O):
+    """A layer with every group on the grouped GEMM, captured into a HIP graph
+    on the context's stream and replayed three times, with eager calls of
+    another batch between the replays: every replay's output equals the eager
+    call's bit for bit, and the eager output matches the oracle."""
     import torch
 
     import spt
@@ -444,18 +441,18 @@ def test_moe_gemm_side_stream_in_graph(O):
                     ctx.forward_moe_batch(cfg, lw, od, oo, 11)
                     stream.synchronize()
                 del g
-        assert_close(ref.cpu().numpy(), O.forward_moe_batch(lay, x, batch, q8=True), what="gemm path, side stream")
+        assert_close(ref.cpu().numpy(), O.forward_moe_batch(lay, x, batch, q8=True), what="gemm path")
     finally:
         ctx.close()
 
 
 def test_moe_batch_beyond_selection_limit(gpu_ctx, O):
-    """A batch of more than 4096 selections runs as slices of whole tokens.
-    The reference fixture at top-2 with 2,100 tokens (4,200 selections:
-    slices of 2,048 and 52 tokens) equals the same tokens sent as those two
-    calls bit for bit, through the device and the host-slice forms, and the
-    oracle within tolerance; at GPT-OSS-120B shape 1,500 tokens (slices of
-    1,024 and 476) equal the two calls bit for bit."""
+    """A batch of more than 8192 selections runs as slices of whole tokens.
+    The reference fixture at top-2 with 4,200 tokens (8,400 selections:
+    slices of 4,096 and 104 tokens) equals the same tokens sent as those two
+    calls bit for bit, through the device, the host-slice and the Q8_0-input
+    forms, and the oracle within tolerance; at GPT-OSS-120B shape 2,300 tokens
+    (slices of 2,048 and 252) equal the two calls bit for bit."""
     import torch
 
     from spt import workloads as W
@@ -463,32 +460,37 @@ def test_moe_batch_beyond_selection_limit(gpu_ctx, O):
     lay = moe_batch_fixture(96, 64, 8, 2, 0, "normal")
     keep, cfg, lw = device_moe_layer(lay)
     H = lay["hidden"]
-    batch = 2100
+    batch = 4200
     x = moe_batch_x(batch, H, "normal")
     xd = torch.from_numpy(x).cuda()
     whole = torch.full((batch * H,), 999.0, dtype=torch.float32, device="cuda")
     parts = torch.full((batch * H,), -999.0, dtype=torch.float32, device="cuda")
     gpu_ctx.forward_moe_batch(cfg, lw, xd, whole, batch)
-    gpu_ctx.forward_moe_batch(cfg, lw, xd[:2048 * H], parts[:2048 * H], 2048)
-    gpu_ctx.forward_moe_batch(cfg, lw, xd[2048 * H:], parts[2048 * H:], batch - 2048)
+    gpu_ctx.forward_moe_batch(cfg, lw, xd[:4096 * H], parts[:4096 * H], 4096)
+    gpu_ctx.forward_moe_batch(cfg, lw, xd[4096 * H:], parts[4096 * H:], batch - 4096)
+    xq = torch.empty(batch * H // 32 * 34, dtype=torch.uint8, device="cuda")
+    gpu_ctx.quantize_q8_0(xd, xq)
+    q8_out = torch.full((batch * H,), 99.0, dtype=torch.float32, device="cuda")
+    gpu_ctx.forward_moe_batch_q8(cfg, lw, xd, xq, q8_out, batch)
     host_out = np.zeros(batch * H, np.float32)
     gpu_ctx.forward_moe_batch_host(cfg, lw, x, host_out, batch)
     torch.cuda.synchronize()
     got = whole.cpu().numpy()
     assert np.array_equal(bits(got), bits(parts.cpu().numpy()))
     assert np.array_equal(bits(got), bits(host_out))
-    assert_close(got, O.forward_moe_batch(lay, x, batch, q8=True, threads=8), what="2,100 tokens")
+    assert np.array_equal(bits(got), bits(q8_out.cpu().numpy()))
+    assert_close(got, O.forward_moe_batch(lay, x, batch, q8=True, threads=8), what="4,200 tokens")
 
     shp = W.MoEShape()
     dl = W.device_layer(gpu_ctx, seed=6, layer=0, shp=shp)
-    batch = 1500
+    batch = 2300
     Hg = shp.hidden
     xg = torch.from_numpy(W.x_tokens(6, 0, batch, Hg)).cuda()
     whole = torch.full((batch * Hg,), 999.0, dtype=torch.float32, device="cuda")
     parts = torch.full((batch * Hg,), -999.0, dtype=torch.float32, device="cuda")
     gpu_ctx.forward_moe_batch(dl.config, dl.layer, xg, whole, batch)
-    gpu_ctx.forward_moe_batch(dl.config, dl.layer, xg[:1024 * Hg], parts[:1024 * Hg], 1024)
-    gpu_ctx.forward_moe_batch(dl.config, dl.layer, xg[1024 * Hg:], parts[1024 * Hg:], batch - 1024)
+    gpu_ctx.forward_moe_batch(dl.config, dl.layer, xg[:2048 * Hg], parts[:2048 * Hg], 2048)
+    gpu_ctx.forward_moe_batch(dl.config, dl.layer, xg[2048 * Hg:], parts[2048 * Hg:], batch - 2048)
     torch.cuda.synchronize()
     got = whole.cpu().numpy()
     assert np.all(np.isfinite(got))

@@ -87,6 +87,68 @@ def test_pack_lists_order(gpu_ctx, O, batch, topk, experts):
     assert np.array_equal(g["list"][:offsets[-1]], lst)
 
 
+@pytest.mark.parametrize("batch,topk,experts", [(2048, 4, 256), (4095, 2, 256), (8191, 1, 37), (8192, 1, 256), (2730, 3, 5),
+                                                (512, 16, 16)])
+@pytest.mark.parametrize("path", ["gemm", "gemv"])
+def test_large_launch_sequence(gpu_ctx, O, batch, topk, experts, path):
+    """Up to 8,192 selections in one launch sequence (lists of more than 64 KB of
+    LDS): every token's output has the bits of calls of at most 4,096 selections
+    (neither path's result depends on an entry's place), and a sample of them the
+    oracle's values."""
+    import torch
+
+    from test_gpu_moe import assert_close, gemm_path
+
+    H, D = 96, 64
+    lay = moe_batch_fixture(H, D, experts, topk, 0, "normal")
+    rng = np.random.default_rng(batch + experts)
+    lay["router"] = rng.standard_normal(experts * H).astype(np.float32)
+    keep, cfg, lw = device_moe_layer(lay)
+    x = rng.standard_normal(batch * H).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    whole, parts = torch.full_like(xd, 5.0), torch.full_like(xd, 7.0)
+    step = 4096 // topk
+    with gemm_path(gpu_ctx, path):
+        gpu_ctx.forward_moe_batch(cfg, lw, xd, whole, batch)
+        for t in range(0, batch, step):
+            n = min(step, batch - t)
+            gpu_ctx.forward_moe_batch(cfg, lw, xd[t * H:(t + n) * H], parts[t * H:(t + n) * H], n)
+        torch.cuda.synchronize()
+    got = whole.cpu().numpy()
+    assert np.array_equal(bits(got), bits(parts.cpu().numpy()))
+    rows = np.unique(np.r_[0:16, rng.integers(0, batch, 64), batch - 16:batch])
+    want = O.forward_moe_batch(lay, np.ascontiguousarray(x.reshape(batch, H)[rows]).reshape(-1), len(rows), q8=True, threads=8)
+    assert_close(got.reshape(batch, H)[rows].reshape(-1), want, what="sample")
+
+
+@pytest.mark.parametrize("off", [1, 3, 10, 15])
+@pytest.mark.parametrize("hidden,dim", [(1472, 96), (96, 1472), (2880, 64)])
+def test_wide_unaligned_experts(gpu_ctx, O, hidden, dim, off):
+    """Expert matrices that begin `off` bytes past a 16-byte boundary give the
+    bits of aligned ones (rows of one part and of two, gate, up and down)."""
+    import torch
+
+    import spt
+    from test_gpu_moe import gemm_path
+
+    lay = moe_batch_fixture(hidden, dim, 3, 2, 0, "normal")
+    keep, cfg, lw = device_moe_layer(lay)
+    x = torch.from_numpy(moe_batch_x(70, hidden, "normal")).cuda()
+    outs = []
+    for o in (0, off):
+        for name, shape in (("gate", [hidden, dim, 3]), ("up", [hidden, dim, 3]), ("down", [dim, hidden, 3])):
+            buf = torch.zeros(lay[name].size + 64, dtype=torch.uint8, device="cuda")
+            buf[o:o + lay[name].size] = torch.from_numpy(lay[name]).cuda()
+            keep[f"{name} {o}"] = buf
+            setattr(lw, f"ffn_{name}_exps", spt.Tensor.make(name, spt.TYPE_MXFP4, shape, buf.data_ptr() + o, lay[name].size))
+        out = torch.full((70 * hidden,), 9.0, device="cuda")
+        with gemm_path(gpu_ctx, "gemm"):
+            gpu_ctx.forward_moe_batch(cfg, lw, x, out, 70)
+            torch.cuda.synchronize()
+        outs.append(bits(out.cpu().numpy()))
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("hidden,experts,batch", [(2880, 128, 771), (96, 37, 2053), (4128, 256, 385)])
 def test_route_wide_bits(gpu_ctx, O, hidden, experts, batch):
     """The large-batch router (8 x 8 logits a wavefront, 384 workgroups and
