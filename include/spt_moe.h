@@ -331,9 +331,9 @@ int spt_forward_moe(struct spt_ctx *ctx, const spt_moe_config *cfg, const spt_mo
  * softmax, per-expert grouping, gate/up, clamped SwiGLU, down and the
  * weighted combine for batch tokens of x [batch][hidden] into out.
  * x and out must not overlap.  Any batch is accepted, as the reference
- * accepts any (moe_batch.go:29-38,84-90): a batch of more than 4096
+ * accepts any (moe_batch.go:29-38,84-90): a batch of more than 8192
  * selections (batch * experts used) runs as consecutive slices of
- * 4096 / experts-used whole tokens (1,024 at top-4), each token's output
+ * 8192 / experts-used whole tokens (2,048 at top-4), each token's output
  * computed from its own row of x as in one call of that slice.  Limits:
  * experts used <= 16 and experts <= 256 (SPT_ERR_INVALID beyond). */
 int spt_forward_moe_batch(struct spt_ctx *ctx, const spt_moe_config *cfg,

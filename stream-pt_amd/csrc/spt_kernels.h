@@ -63,7 +63,7 @@ struct SelectOut {
 constexpr int kGvStartMax = 512;
 constexpr int kGvStartWords = 8;
 
-// Optional Q8_0 outputs of a quantized activation (see write_q8_block);
+// Optional Q8_0 outputs of a quantized activation (see write_q8_lane);
 // with src34 set, the router's launch unpacks these GGML Q8_0 blocks of the
 // input instead of quantizing it.
 struct QuantOut {

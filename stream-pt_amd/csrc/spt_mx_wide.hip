@@ -24,10 +24,10 @@
 // about 64 entries the weight stream (HBM) is the floor, and beyond it the
 // one FMA per output and block (16 per MFMA and lane, twice the MFMA's own
 // cycles).  Measured at GPT-OSS-120B shape, gate/up + down: 2,000 tokens
-// (8,000 selections, 62 per expert) 586 + 271 us, 0.46 PFLOP/s, 1.9 TB/s of
+// (8,000 selections, 62 per expert) 588 + 265 us, 0.47 PFLOP/s, 1.9 TB/s of
 // weights; the bf16 MFMA form it replaces (16-row fragments, the weights in
 // 96-byte row windows) took 1,016 + 462 us in the two slices it ran as; 512
-// tokens, Zipf(1.1): the layer 452 -> 415 us.  Of a step's 10,000 cycles per
+// tokens, Zipf(1.1): the layer 452 -> 412 us.  Of a step's 10,000 cycles per
 // compute unit the products take half, the waves' sums and the epilogue a
 // quarter, waiting for loads the rest.
 
