@@ -360,7 +360,10 @@ int spt_forward_moe_batch_q8(struct spt_ctx *ctx, const spt_moe_config *cfg, con
                              const float *x_dev, const void *xq_dev, int64_t x_len, float *out_dev,
                              int64_t out_len, int64_t batch);
 
-/* forwardMoEBatch (spt_forward_moe_batch, same results bit for bit) for
+/* forwardMoEBatch (spt_forward_moe_batch, same results bit for bit; within
+ * the fp32 tolerance where expert biases begin between elements and their
+ * aligned copies do not fit the array, which keeps such a batch off the
+ * grouped GEMM) for
  * callers that cannot allocate: code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc.  No reference counterpart.  It
  * calls no hipMalloc / hipFree and records no timing events: its scratch is
