@@ -368,7 +368,7 @@ int spt_forward_moe_batch_q8(struct spt_ctx *ctx, const spt_moe_config *cfg, con
  * loops, harnesses that forbid hipMalloc.  No reference counterpart.  It
  * calls no hipMalloc / hipFree and records no timing events: its scratch is
  * a fixed 32 MiB device array, one per GPU, held until the process ends
- * (about 91 KB per token at GPT-OSS-120B shape below 256 tokens, 120 KB from
+ * (about 91 KB per token at GPT-OSS-120B shape below 96 tokens, 120 KB from
  * there: batches up to about 270 tokens); larger batches fail with
  * SPT_ERR_INVALID.  Every call on a GPU uses that GPU's one array, so calls
  * that overlap on one GPU (several contexts, streams or threads) race; a
