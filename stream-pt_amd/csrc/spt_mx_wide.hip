@@ -213,9 +213,10 @@ __device__ float lut_dot(const ByteView &v, uint32_t row_pos, int nb, const int8
 //
 // The waves' partial sums of a step meet in LDS, and each output's partials
 // (eight, or four with RT = 2) are added in wave order, so it does not depend
-// on its entry's place in the list.  A wave takes eight entries of a two-tile pass (four of
-// a one-tile pass), all 32 rows of a tile, so a 32-element Q8_0 block of act stays
-// within it.  This epilogue of a step runs at the start of the next one.
+// on its entry's place in the list.  A wave takes eight entries of a two-tile
+// pass (four of a one-tile pass), all 32 rows of a tile, so a 32-element Q8_0
+// block of act stays within it.  This epilogue of a step runs at the start of
+// the next one.
 template <int MODE, int P, int NJ, int RT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_mx_wide(MxWideArgs) {
     constexpr int kSub = MODE == kGateUp ? 2 : 1;  // steps per unit
